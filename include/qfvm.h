@@ -303,10 +303,12 @@ int qfvm_profile_json(qfvm_handle h, char* buf, int64_t cap, int64_t* len, int32
 /*
  * Execution options of one handle (no counterpart in the reference). Keys:
  *   "fusion"      1 = plan gates into fused LDS-tiled passes (default), 0 = one kernel per gate
- *   "tile_bits"   qubits per fused tile b (4..14; 0 = default: 11 for complex128, 12 for complex64;
+ *   "tile_bits"   qubits per fused tile b (4..14; 0 = default: 12 for matrix-core passes, else 11 for
+ *                 complex128, 12 for complex64;
  *                 the adjoint's two-state sweep uses b - 1 of an explicit value, 11 / 12 by default)
- *   "low_bits"    low qubits always in a tile L (0 = default: 5 for one-state passes, 6 for two-state)
- *   "max_groups"  4-qubit register groups per fused pass (1..24, default 12)
+ *   "low_bits"    low qubits always in a tile L (0 = default: 4 for matrix-core passes, 3 at complex128
+ *                 up to 25 qubits; else 5 for one-state passes, 6 for two-state)
+ *   "max_groups"  register groups (of 3 or 4 qubits) per fused pass (1..24, default 12)
  *   "pass_cost"   compute budget of one fused pass in quarter dense-gate units (0 = default)
  *   "split_rows"  1 = (default) complex128 one-state passes of 2^10..2^13-amplitude tiles and the
  *                 two-state passes of the adjoint (both precisions, 2^10 to 2^12 per state) run
@@ -320,18 +322,22 @@ int qfvm_profile_json(qfvm_handle h, char* buf, int64_t cap, int64_t* len, int32
  *                 8-amplitude row (3-qubit groups) per lane instead of split rows, 0 = split rows
  *   "rows8_c64"   1 = complex64 one-state passes of such tiles do the same (with "rows8" on),
  *                 0 = (default) 16-amplitude rows
- *   "layout"      1 = layout-aware planning of those row-of-8 passes: a pass may store its tile with
- *                 its qubits in other places (the tile's addresses stay the same), so that the qubits
- *                 the next passes act on sit in the low positions every tile holds; fewer passes per
- *                 circuit, and passes without gates at the end of each call restore the qubit order,
- *                 so the state between calls is always in the standard order. 0 = (default) off
+ *   "layout"      layout-aware planning of one-state passes: a pass may store its tile with its qubits
+ *                 in other places (the tile's addresses stay the same), so that the qubits the next
+ *                 passes act on sit in the low positions every tile holds; fewer passes per circuit,
+ *                 and the qubits are back in order at the end of each call, so the state between
+ *                 calls is always in the standard order. 1 = on, 0 = off; by default it is on for
+ *                 matrix-core passes (see "mfma") and off for the others
  *   "stream"      1 = persistent fused-pass kernel that prefetches the next tile (complex128,
  *                 one-state passes of 2^11..2^13-amplitude tiles, when split_rows does not apply),
  *                 0 = one workgroup per tile
  *   "stagger"     persistent kernel: start delay of half the workgroups, in 8128-cycle sleeps (0..64)
  *   "stagger_shift" the blockIdx bit that selects the delayed half (0..16)
- *   "mfma"        1 = (default) dense gates on 4 to 8 targets run on the matrix cores (FP64 MFMA at
- *                 complex128, FP32 MFMA at complex64), 0 = on the vector ALUs
+ *   "mfma"        1 = (default) dense gates on 4 to 8 targets and, with "rows8" on, the groups of
+ *                 complex128 one-state passes (2^9 to 2^13-amplitude tiles with 128-byte runs or
+ *                 longer; gate lists that are mostly controlled phases keep the vector kernels where
+ *                 those take less time) run on the matrix cores (FP64 MFMA at complex128, FP32 MFMA at
+ *                 complex64), 0 = on the vector ALUs
  *   "dense_blocks" k (0 = off, or 4..8; default 5): qfvm_apply and qfvm_run (not qfvm_adjoint) on
  *                 states of 14 or more qubits with "mfma" on collapse runs of gates confined to at
  *                 most k qubits into one dense gate

@@ -32,7 +32,7 @@ DEVICE += ["-mllvm", "-simplifycfg-sink-common=false"]
 # at every join (measured on the row-of-8 kernel: 112 instead of 122 VGPRs, 30% fewer moves).
 DEVICE += ["-mllvm", "-structurizecfg-skip-uniform-regions"]
 
-SOURCES = ["gates.hip", "reduce.hip", "sample.hip", "fused.hip", "plan.cpp", "capi.cpp"]
+SOURCES = ["gates.hip", "reduce.hip", "sample.hip", "fused.hip", "pass_mat.hip", "plan.cpp", "capi.cpp"]
 
 
 def _compile(src: str) -> str:

@@ -1195,20 +1195,14 @@ int qfvm_plan_json(int32_t n, int32_t dtype, int32_t tile_bits, int32_t low_bits
         // collapsed when asked
         gates = merge_single_qubit_runs(gates);
         if (dense_blocks) gates = collapse_dense_blocks(gates, dense_blocks, dense_min_gates > 0 ? dense_min_gates : 24);
-        FuseConfig cfg;
-        cfg.tile_bits = tile_bits > 0 ? tile_bits : default_tile_bits(tmp.dtype, 1);
-        cfg.low_bits = low_bits > 0 ? low_bits : default_low_bits(tmp.dtype, 1);
+        tmp.tile_bits = tile_bits;
+        tmp.low_bits = low_bits;
+        tmp.layout = layout != 0;
+        FuseConfig cfg = circuit_config(tmp, gates);  // with default options, as qfvm_apply
+        if (tile_bits > 0 && tile_bits < cfg.tile_bits) cfg.tile_bits = tile_bits;
         cfg.max_groups = max_groups > 0 ? max_groups : 12;
         cfg.max_cost = pass_cost > 0 ? pass_cost : 0;
-        // the group width qfvm_apply would use with default options (complex128: rows of 8)
-        const int bb = std::min(cfg.tile_bits, n);
-        if (tmp.dtype == QFVM_C128 && bb >= 10 && bb <= 13) cfg.group_bits = 3;
-        // complex64 gate lists with dense 2-target gates take the row-of-8 kernel (as qfvm_apply)
-        if (tmp.dtype == QFVM_C64 && bb >= 10 && bb <= 13)
-            for (const Gate& g : gates)
-                if (g.kind == G_MULTI && g.targets.size() == 2) cfg.group_bits = 3;
-        cfg.layout = layout != 0 && cfg.group_bits == 3;
-        std::vector<PlanItem> plan = plan_gates(gates, n, cfg);
+        std::vector<PlanItem> plan = plan_circuit(gates, n, cfg);
         std::string j = "{\"items\": [";
         char t[512];
         auto cplx = [&](const cd& z) {

@@ -84,6 +84,7 @@ struct FPass {
     std::vector<int> Q;          // tile qubits, ascending; Q[0..L-1] = 0..L-1
     std::vector<FGroup> groups;
     int group_bits = FUSE_GROUP_BITS;  // qubits per compute group (3: rows of 8, 4: rows of 16)
+    bool mat = false;  // matrix-core pass: every group is applied as 8x8 matrices (pass_mat.hip)
     // layout-aware plans: the pass stores local bit k of its tile at local bit out_bit[k] (a
     // permutation of 0..b-1; empty = in place). The tile's addresses do not change, only which
     // qubit each of its address bits stands for.
@@ -97,7 +98,17 @@ struct FuseConfig {
     int max_cost;    // compute budget of a pass in quarter dense-gate units (0: unlimited)
     int group_bits = FUSE_GROUP_BITS;  // qubits per compute group: 3 or 4
     bool layout = false;  // layout-aware planning (row-of-8 one-state passes only, see plan.cpp)
+    bool mat = false;     // groups for the matrix-core pass kernel: at most mat_ext(b) outside qubits each
+    // with mat: the shape of a plan on the vector kernels, for gate lists that suit those better
+    int vec_tile_bits = 0, vec_low_bits = 0, vec_group_bits = 0;
+    bool vec_layout = false;
 };
+
+// Outside qubits (controls and diagonal targets that are not group qubits) one group of a matrix-core
+// pass may depend on: the group has one 8x8 matrix per value of them, picked per 32 rows, so the ones
+// inside the tile must be row bits that the 32 rows of two matrix products share (b - 8 of the b - 3).
+constexpr int MAT_MAX_EXT = 4;
+inline int mat_ext(int b) { return b - 8 < MAT_MAX_EXT ? b - 8 : MAT_MAX_EXT; }
 
 // Default tile shape per precision and state count (states = 2: the adjoint's two-state sweep, both
 // tiles in LDS). complex128: 2^11-amplitude tiles, which let four workgroups share a CU (faster than
@@ -116,6 +127,10 @@ struct PlanItem {
     std::vector<int> l2p;  // single gates in layout-aware plans: position of each qubit (empty = identity)
 };
 
+// the configuration a gate list of qfvm_apply / qfvm_run is planned with
+FuseConfig circuit_config(const State& s, const std::vector<Gate>& gates);
+// plan_gates, for cfg.mat on the better of the two kinds of passes (the choice shows in FPass::mat)
+std::vector<PlanItem> plan_circuit(const std::vector<Gate>& gates, int n, const FuseConfig& cfg);
 std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const FuseConfig& cfg);
 // Runs of uncontrolled one-qubit gates on one qubit (no other gate on that qubit between them)
 // merged into one gate each: diagonal if every factor is, real if every factor is real, else dense;
@@ -135,5 +150,7 @@ const std::vector<PlanItem>& cached_plan(State& s, const std::vector<Gate>& gate
 // `lam` set, every gate acts on both s.psi and lam (the reverse sweep) and the plan's gradient
 // markers write grads_dev[slot].
 void execute_plan(State& s, const std::vector<PlanItem>& plan, void* lam = nullptr, double* grads_dev = nullptr);
+// Runs a plan of matrix-core passes (pass_mat.hip); execute_plan calls it for those.
+void execute_mat_plan(State& s, const std::vector<PlanItem>& plan);
 
 }  // namespace qfvm

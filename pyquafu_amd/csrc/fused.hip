@@ -2083,6 +2083,12 @@ static void execute_typed(State& s, const std::vector<PlanItem>& plan, void* lam
 }
 
 void execute_plan(State& s, const std::vector<PlanItem>& plan, void* lam, double* grads_dev) {
+    for (const PlanItem& it : plan)
+        if (it.fused && it.pass.mat) {
+            if (lam) throw Error(QFVM_ERR_RUNTIME, "matrix-core passes act on one state");
+            execute_mat_plan(s, plan);
+            return;
+        }
     if (lam) {
         if (s.dtype == QFVM_C128)
             execute_typed<double, 2>(s, plan, lam, grads_dev);

@@ -411,7 +411,28 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
             info[i].multi = false;
             info[i].dense2 = true;
         }
+        // a gate of more qubits than a matrix-core group and its outside qubits hold (or, in tiles with
+        // few free qubits, of more controls than it may leave outside) runs by itself
+        if (cfg.mat && !info[i].multi && popc(info[i].D) > mat_ext(b) &&
+            (popc(info[i].N | info[i].D) > gb + mat_ext(b) || (b < n && b - L < gb)))
+            info[i].multi = true;
     }
+    // Whether a gate on A (non-diagonal on N) can join a matrix-core group on S that touches GA, and the
+    // group's qubits then: outside qubits beyond the limit become group qubits, if the tile Q (widened
+    // if need be) and the group have room.
+    auto join = [&](uint64_t& S, uint64_t GA, uint64_t N, uint64_t A, uint64_t& Q) {
+        S |= N;
+        for (;;) {
+            const uint64_t ext = (GA | A) & ~S;
+            if (popc(S) > gb) return false;
+            if (popc(ext) <= mat_ext(b)) return true;
+            const uint64_t in = ext & Q;
+            const uint64_t q = in ? in & -in : ext & -ext;
+            if (!in && popc(Q) >= b) return false;
+            Q |= q;
+            S |= q;
+        }
+    };
     std::vector<char> done(gates.size(), 0);
     std::vector<PlanItem> plan;
     size_t first = 0;
@@ -440,21 +461,38 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
             uint64_t newQ = Q | g.N;
             if (take && popc(newQ) > b) take = false;
             int place = -1;
+            uint64_t placeS = 0;  // matrix-core passes: the group's qubits with the gate
             if (take) {
                 // latest group that can hold the gate (a stage holds markers, a compute group gates),
-                // moving back only past groups it commutes with
+                // moving back only past groups it commutes with. Matrix-core passes: the group that
+                // the gate widens least (new group qubits, then new outside qubits), the latest of equals
+                int widen = 1 << 20;
+                const uint64_t baseQ = newQ;
                 for (int j = (int)groups.size() - 1; j >= 0; j--) {
                     const GroupB& G = groups[j];
-                    const bool fits = g.grad ? G.stage
-                                             : (!G.stage && ((G.S & g.N) == g.N || popc(G.S | g.N) <= gb));
+                    uint64_t Q1 = baseQ, S1 = G.S;
+                    const bool fits = cfg.mat  ? join(S1, G.A, g.N, A, Q1)
+                                      : g.grad ? G.stage
+                                               : (!G.stage && ((G.S & g.N) == g.N || popc(G.S | g.N) <= gb));
                     if (fits) {
-                        place = j;
-                        break;
+                        const int w = cfg.mat ? 4 * popc(S1 & ~G.S) + std::max(0, popc((G.A | A) & ~S1) - popc(G.A & ~G.S)) : 0;
+                        if (w < widen) {
+                            widen = w;
+                            place = j;
+                            placeS = S1;
+                            newQ = Q1;
+                        }
+                        if (w == 0) break;
                     }
                     if (!commutes(g, G)) break;  // cannot move before group j
                 }
                 if (place < 0) {
-                    if ((int)groups.size() < cfg.max_groups) {
+                    if (cfg.mat) {
+                        newQ = baseQ;
+                        placeS = 0;
+                        take = join(placeS, 0, g.N, A, newQ);
+                    }
+                    if (take && (int)groups.size() < cfg.max_groups) {
                         groups.emplace_back();
                         groups.back().stage = g.grad;
                         place = (int)groups.size() - 1;
@@ -479,17 +517,24 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
                 continue;
             }
             GroupB& G = groups[place];
-            if (!G.stage) G.S |= g.N;
+            if (!G.stage) G.S |= cfg.mat ? placeS : g.N;
             G.N |= g.N;
             G.A |= A;
             G.gates.push_back((int)i);
             Q = newQ;
             done[i] = 1;
         }
-        // finalize: pad the tile to b qubits and every group to gb tile qubits
+        // finalize: pad the tile to b qubits and every group to gb tile qubits. Matrix-core passes whose
+        // qubits are out of place take misplaced positions with their qubits' homes first
+        if (moved && cfg.mat)
+            for (int p = L; p < n; p++) {
+                const uint64_t add = (1ull << p) | (1ull << phys[(size_t)p]);
+                if (inv[(size_t)p] != p && popc(Q | add) <= b) Q |= add;
+            }
         for (int q = 0; q < n && popc(Q) < b; q++) Q |= 1ull << q;
         PlanItem it{true, FPass{}, Gate{}};
         it.pass.group_bits = gb;
+        it.pass.mat = cfg.mat;
         for (int q = 0; q < n; q++)
             if ((Q >> q) & 1) it.pass.Q.push_back(q);
         for (GroupB& G : groups) {
@@ -511,6 +556,11 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
                 it.pass.groups.push_back(std::move(fg));
                 continue;
             }
+            if (cfg.mat)  // outside qubits of the tile first: each halves the group's matrices
+                for (int q : it.pass.Q) {
+                    if (popc(G.S) >= gb) break;
+                    if ((G.A >> q) & 1) G.S |= 1ull << q;
+                }
             for (int q : it.pass.Q) {
                 if (popc(G.S) >= gb) break;
                 G.S |= 1ull << q;
@@ -527,6 +577,10 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
             for (int gi : G.gates) {
                 FOpHost o = convert(move_gate(gates[gi], cur), info[gi], fg.S);
                 o.src = gi;
+                if (cfg.mat) {  // the group's matrices take every gate as it is
+                    fg.ops.push_back(o);
+                    continue;
+                }
                 // a 4x4 reads its two target bits as they are in memory: their pending relabelings
                 // are applied first, as for controls
                 const uint32_t flush_bits = o.cm_group | (o.kind == F_DENSE4 ? (1u << o.g) | (1u << o.target) : 0u);
@@ -563,7 +617,7 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
             }
             for (int j = 0; j < FUSE_GROUP_BITS; j++) fg.pxm[j] = M[j];
             fg.pxc = C;
-            mark_diagonal_runs(fg);
+            if (!cfg.mat) mark_diagonal_runs(fg);
             it.pass.groups.push_back(std::move(fg));
         }
         if (lay) {
@@ -583,19 +637,52 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
             std::vector<int> order((size_t)bb);
             for (int k = 0; k < bb; k++) order[(size_t)k] = k;
             std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return nxt[(size_t)x] < nxt[(size_t)y]; });
-            std::vector<char> chosen((size_t)bb, 0);
-            for (int k = 0; k < L; k++) chosen[(size_t)order[(size_t)k]] = 1;
             std::vector<int> out((size_t)bb);
             for (int k = 0; k < bb; k++) out[(size_t)k] = k;
-            int lo = 0;
             bool any = false;
-            for (int k = L; k < bb; k++) {
-                if (!chosen[(size_t)k]) continue;
-                while (chosen[(size_t)lo]) lo++;  // a low slot whose qubit is not chosen (one exists per mover)
-                out[(size_t)k] = lo;
-                out[(size_t)lo] = k;
-                lo++;
-                any = true;
+            if (cfg.mat) {
+                // the other qubits go home where their home is in the tile and free, so that few
+                // passes (mostly none) are left to restore the order at the end; qubits without a
+                // later use count as others
+                std::vector<int> at((size_t)n, -1), from((size_t)bb, -1);
+                for (int k = 0; k < bb; k++) at[(size_t)Qv[(size_t)k]] = k;
+                std::vector<char> placed((size_t)bb, 0);
+                auto put = [&](int k, int to) {
+                    out[(size_t)k] = to;
+                    from[(size_t)to] = k;
+                    placed[(size_t)k] = 1;
+                };
+                auto home = [&](int k) { return at[(size_t)inv[(size_t)Qv[(size_t)k]]]; };
+                std::vector<int> low;
+                for (int k = 0; k < L; k++)
+                    if (nxt[(size_t)order[(size_t)k]] < gates.size()) low.push_back(order[(size_t)k]);
+                for (int k : low)
+                    if (home(k) >= 0 && home(k) < L) put(k, home(k));
+                for (int k : low)
+                    if (!placed[(size_t)k] && k < L && from[(size_t)k] < 0) put(k, k);
+                for (int k : low)
+                    for (int to = 0; to < L && !placed[(size_t)k]; to++)
+                        if (from[(size_t)to] < 0) put(k, to);
+                for (int k = 0; k < bb; k++)
+                    if (!placed[(size_t)k] && home(k) >= 0 && from[(size_t)home(k)] < 0) put(k, home(k));
+                for (int k = 0; k < bb; k++)
+                    if (!placed[(size_t)k] && from[(size_t)k] < 0) put(k, k);
+                for (int k = 0; k < bb; k++)
+                    for (int to = 0; to < bb && !placed[(size_t)k]; to++)
+                        if (from[(size_t)to] < 0) put(k, to);
+                for (int k = 0; k < bb; k++) any = any || out[(size_t)k] != k;
+            } else {
+                std::vector<char> chosen((size_t)bb, 0);
+                for (int k = 0; k < L; k++) chosen[(size_t)order[(size_t)k]] = 1;
+                int lo = 0;
+                for (int k = L; k < bb; k++) {
+                    if (!chosen[(size_t)k]) continue;
+                    while (chosen[(size_t)lo]) lo++;  // a low slot whose qubit is not chosen (one exists per mover)
+                    out[(size_t)k] = lo;
+                    out[(size_t)lo] = k;
+                    lo++;
+                    any = true;
+                }
             }
             if (any) {
                 std::vector<int> was((size_t)bb);
@@ -627,6 +714,7 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
         for (int q = 0; q < n && popc(Qm) < b; q++) Qm |= 1ull << q;
         PlanItem it{true, FPass{}, Gate{}};
         it.pass.group_bits = gb;
+        it.pass.mat = cfg.mat;
         std::vector<int> loc((size_t)n, -1);
         for (int q = 0; q < n; q++)
             if ((Qm >> q) & 1) {
@@ -690,7 +778,8 @@ void plan_signature(const std::vector<Gate>& gates, int n, const FuseConfig& cfg
     sig.reserve(gates.size() * 5 + 2);
     sig.push_back((uint64_t)n | ((uint64_t)cfg.tile_bits << 8) | ((uint64_t)cfg.low_bits << 16) |
                   ((uint64_t)cfg.max_groups << 24) | ((uint64_t)cfg.group_bits << 32));
-    sig.push_back((uint64_t)(uint32_t)cfg.max_cost | ((uint64_t)cfg.layout << 32));
+    sig.push_back((uint64_t)(uint32_t)cfg.max_cost | ((uint64_t)cfg.layout << 32) | ((uint64_t)cfg.mat << 33) |
+                  ((uint64_t)cfg.vec_tile_bits << 34) | ((uint64_t)cfg.vec_low_bits << 42) | ((uint64_t)cfg.vec_group_bits << 50) | ((uint64_t)cfg.vec_layout << 54));
     for (const Gate& g : gates) {
         const GInfo gi = info_of(g);
         const uint64_t cls = (gi.diag ? 1u : 0u) | (gi.multi ? 2u : 0u) | (gi.grad ? 4u : 0u) |
@@ -760,7 +849,7 @@ const std::vector<PlanItem>& cached_plan(State& s, const std::vector<Gate>& gate
             if (pc.entries[k].last < pc.entries[old].last) old = k;
         pc.entries.erase(pc.entries.begin() + (std::ptrdiff_t)old);
     }
-    pc.entries.push_back(PlanCache::Entry{h, pc.sig, plan_gates(gates, s.n, cfg), pc.clock});
+    pc.entries.push_back(PlanCache::Entry{h, pc.sig, plan_circuit(gates, s.n, cfg), pc.clock});
     s.kstats[(size_t)s.stat_index("plan_cache_miss")].second.launches++;
     return pc.entries.back().plan;
 }
@@ -777,7 +866,7 @@ static FuseConfig config_of(const State& s, int states) {
     // and complex64 with option "rows8_c64"
     const int b = std::min(cfg.tile_bits, s.n);
     if (states == 1 && s.rows8 && (s.dtype == QFVM_C128 || s.rows8_c64) && b >= 10 && b <= 13) cfg.group_bits = 3;
-    cfg.layout = s.layout && cfg.group_bits == 3;
+    cfg.layout = s.layout > 0 && cfg.group_bits == 3;
     return cfg;
 }
 
@@ -795,28 +884,83 @@ void apply_circuit(State& s, const std::vector<Gate>& gates_in) {
         apply_gates(s, gates);
 }
 
+// One-state plans on the vector kernels: complex64 runs rows of 16 by default; a gate list with dense
+// 2-target gates takes the row-of-8 kernel instead, whose passes hold those gates (each would
+// otherwise cost a sweep).
+static FuseConfig vector_config(const State& s, const std::vector<Gate>& gates) {
+    FuseConfig cfg = config_of(s, 1);
+    const int b = std::min(cfg.tile_bits, s.n);
+    if (cfg.group_bits != 3 && s.rows8 && s.dtype == QFVM_C64 && b >= 10 && b <= 13) {
+        for (const Gate& g : gates)
+            if (g.kind == G_MULTI && g.targets.size() == 2) {
+                cfg.group_bits = 3;
+                cfg.layout = s.layout > 0;
+                break;
+            }
+    }
+    return cfg;
+}
+
+// Matrix-core passes (complex128) take tiles of 2^9 to 2^13 amplitudes in contiguous runs of 8 or more.
+// Tiles of 2^12 by default: eight more qubits than the low four (three up to 25 qubits, where a run of
+// 128 bytes costs less than the passes it saves). Swept over tiles of 2^9..2^13 and 3..5 low bits at 10
+// to 28 qubits, this is within 8% of the best shape everywhere.
+FuseConfig circuit_config(const State& s, const std::vector<Gate>& gates) {
+    const FuseConfig vec = vector_config(s, gates);
+    if (!s.rows8 || !s.mfma || s.dtype != QFVM_C128) return vec;
+    FuseConfig cfg = vec;
+    cfg.mat = true;
+    cfg.group_bits = 3;
+    cfg.layout = s.layout != 0;
+    cfg.vec_layout = vec.layout;
+    cfg.vec_tile_bits = vec.tile_bits;
+    cfg.vec_low_bits = vec.low_bits;
+    cfg.vec_group_bits = vec.group_bits;
+    if (s.tile_bits == 0) cfg.tile_bits = 12;
+    if (s.low_bits == 0) cfg.low_bits = s.n <= 25 ? 3 : 4;
+    const int b = std::min(cfg.tile_bits, s.n);
+    const int low = b < s.n ? std::min(cfg.low_bits, b - 1) : b;
+    return b >= 9 && b <= 13 && low >= 3 ? cfg : vec;
+}
+
+std::vector<PlanItem> plan_circuit(const std::vector<Gate>& gates, int n, const FuseConfig& cfg) {
+    if (!cfg.mat) return plan_gates(gates, n, cfg);
+    FuseConfig v = cfg;
+    v.mat = false;
+    v.tile_bits = cfg.vec_tile_bits;
+    v.low_bits = cfg.vec_low_bits;
+    v.group_bits = cfg.vec_group_bits;
+    v.layout = cfg.vec_layout;
+    // a handful of gates (the runs between noise channels) is over before its matrices are built (10 us)
+    if (gates.size() < 8) return plan_gates(gates, n, v);
+    std::vector<PlanItem> plan = plan_gates(gates, n, cfg);
+    // Gate lists that are mostly diagonal gates between qubits far apart (a QFT: every pair) need many
+    // groups, since a group depends on few outside qubits, while the vector kernels merge any number
+    // of them into one angle per row. Measured at 28 qubits, complex128: a matrix-core pass takes
+    // 1.6 ms plus 0.11 ms per group, a vector pass of a QFT 2.0 ms.
+    // Gates with many controls run one by one between matrix-core passes but inside vector passes.
+    size_t diag = 0, single = 0;
+    for (const Gate& g : gates) diag += info_of(g).N == 0;
+    for (const PlanItem& it : plan) single += !it.fused && it.gate.kind != G_MULTI;
+    if (diag <= 2 * (gates.size() - diag) && single == 0) return plan;
+    std::vector<PlanItem> vec = plan_gates(gates, n, v);
+    double cm = 0.0, cv = 0.0;
+    for (const PlanItem& it : plan) cm += it.fused ? 1.0 + 0.07 * (double)it.pass.groups.size() : 1.0;
+    for (const PlanItem& it : vec) cv += it.fused ? 1.25 : 1.0;
+    return cm <= cv ? plan : vec;
+}
+
 void apply_gates(State& s, const std::vector<Gate>& gates) {
     if (gates.empty()) return;
     if (!s.fusion || s.n < 6) {
         for (const Gate& g : gates) launch_gate(s, g);
         return;
     }
-    FuseConfig cfg = config_of(s, 1);
-    // complex64 runs rows of 16 by default; a gate list with dense 2-target gates takes the
-    // row-of-8 kernel instead, whose passes hold those gates (each would otherwise cost a sweep)
-    const int b = std::min(cfg.tile_bits, s.n);
-    if (cfg.group_bits != 3 && s.rows8 && s.dtype == QFVM_C64 && b >= 10 && b <= 13) {
-        for (const Gate& g : gates)
-            if (g.kind == G_MULTI && g.targets.size() == 2) {
-                cfg.group_bits = 3;
-                cfg.layout = s.layout;
-                break;
-            }
-    }
+    const FuseConfig cfg = circuit_config(s, gates);
     if (s.plan_cache_on)
         execute_plan(s, cached_plan(s, gates, cfg));
     else
-        execute_plan(s, plan_gates(gates, s.n, cfg));
+        execute_plan(s, plan_circuit(gates, s.n, cfg));
 }
 
 void apply_gates2(State& s, const std::vector<Gate>& gates, void* lam, double* grads_dev) {
