@@ -269,7 +269,7 @@ struct PauliHost {
     int slot;
 };
 constexpr int EXPECT_BATCH = 256;
-constexpr size_t EXPECT_PARTIALS = 32 * 2048;
+constexpr size_t EXPECT_PARTIALS = (size_t)(EXPECT_BATCH + 4 * 24) * 512;
 constexpr size_t RED_PARTIALS = 2048 + 1;
 void queue_expectations(State& s, const PauliHost* terms, int n_terms, double* out_dev, double* partials,
                         double* fallback, bool account = true);

@@ -341,6 +341,196 @@ __global__ void __launch_bounds__(RED_BLOCK) k_term_sums(const double* __restric
 }
 
 // ------------------------------------------------------------------------------------------------
+// Expectations of Z strings and single-qubit X / Y letters (fields, Bloch vectors, Ising energies): the
+// same tiles, but every sum a term can need is taken at once, so a term costs nothing per amplitude.
+//   * X and Y of every tile qubit: the tile's bits fall into four groups of three; a thread gathers the 8
+//     amplitudes that differ in a group's bits and adds Re and Im of psi[i] conj(psi[i ^ bit]) of its
+//     four pairs per bit to one of 24 accumulators.
+//   * Z strings: the tile's probabilities take a Walsh-Hadamard transform, three bits at a time in
+//     registers; entry m of it is the sum of (-1)^popc(i & m) |psi_i|^2 over the tile. Thread k reads the
+//     entry of string k's bits and signs it by the string's bits outside the tile. All strings go to the
+//     first pass.
+// What bounds it: its reads of the state, with the LDS close behind (four gathers of the tile for the flips,
+// three more for the transform). Tiles of 2^12 amplitudes in runs of 128 bytes hold 9 (complex128) or 8
+// (complex64) chosen qubits: 3 reads for the fields of 27 to 30 qubits, where the tiles of general
+// strings (2^11 amplitudes, runs of 32, one accumulator per term) take 4 or 5. Measured on 27 qubits at
+// complex128, 27 ZZ bonds and 27 X fields: 2.62 ms -> 1.31 ms; 27 Z terms alone one read of 0.36 ms, 5.9 TB/s.
+constexpr int FT_BITS = 12;        // tile bits; smaller states are padded with zeros
+constexpr int FT_THREADS = 1 << (FT_BITS - 3);
+constexpr unsigned FT_GRID = 512;  // two workgroups per CU
+constexpr int FT_COLS = 24;        // X and Y columns of a pass (bit k: columns 2 k and 2 k + 1)
+
+struct FPassArg {
+    int size_bits;           // qubits of the state
+    int nz;                  // Z strings of the pass
+    uint32_t need;           // bit 2 g: some X on group g's bits is asked for, bit 2 g + 1: some Y
+    uint32_t smask[12], sshift[12];  // tile t sits at the offset sum of (t & smask[i]) << sshift[i]
+    uint8_t q[FT_BITS];      // tile qubits, ascending
+    uint8_t row[4][FT_BITS - 3];      // per group: the tile bits that the thread index's bits stand for
+    uint64_t z[EXPECT_BATCH];    // strings, global bits
+    uint16_t zl[EXPECT_BATCH];   // and tile-local bits
+};
+static_assert(EXPECT_BATCH <= FT_THREADS, "a thread per string");
+static_assert(sizeof(FPassArg) <= 3072, "kernel argument size");
+
+// LDS slot of tile-local element l: the low bits XORed by the higher ones, three (16-byte elements) or
+// four (8 bytes) at a time, so that the rows of any group spread over all banks (linear over XOR)
+template <int BYTES>
+__host__ __device__ constexpr int ft_slot(int l) {
+    return BYTES == 16 ? l ^ (((l >> 3) ^ (l >> 6) ^ (l >> 9)) & 7) : l ^ (((l >> 4) ^ (l >> 8)) & 15);
+}
+
+// Workgroups walk the tiles. partials: column c's value of each workgroup. STRINGS: with Z strings
+template <typename R, bool STRINGS>
+__global__ void __launch_bounds__(FT_THREADS, 4) k_expect_fields(const V2<R>* __restrict__ psi, const FPassArg pp,
+                                                          uint64_t tiles, double* __restrict__ partials) {
+    extern __shared__ unsigned char lds_raw[];
+    constexpr int ES = (int)sizeof(V2<R>);
+    V2<R>* tile = reinterpret_cast<V2<R>*>(lds_raw);
+    double* prob = reinterpret_cast<double*>(lds_raw);  // the same memory, after the amplitudes are done
+    const int tid = threadIdx.x;
+    constexpr int NTH = FT_THREADS, b = FT_BITS;
+    const uint64_t size = 1ull << pp.size_bits;
+    const bool string = STRINGS && tid < pp.nz;
+    double az = 0.0;
+    int row[4];  // local index of member 0 of this thread's row, per group
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        row[g] = 0;
+        for (int k = 0; k < b - 3; k++) row[g] |= ((tid >> k) & 1) << pp.row[g][k];
+    }
+    uint64_t l2g = 0;
+    for (int k = 0; k < b - 3; k++) l2g |= (uint64_t)((tid >> k) & 1) << pp.q[k];
+    const uint64_t t0 = 1ull << pp.q[b - 3], t1 = 1ull << pp.q[b - 2], t2 = 1ull << pp.q[b - 1];
+    double re[4][3], im[4][3];
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) re[g][k] = im[g][k] = 0.0;
+    for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+        // (opaque per tile: hoisted out of the loop, the slots of all rows would not fit the registers)
+        asm volatile("" : "+v"(row[0]), "+v"(row[1]), "+v"(row[2]), "+v"(row[3]), "+v"(l2g));
+        uint64_t base = 0;
+#pragma unroll
+        for (int k = 0; k < 12; k++) base |= (t & pp.smask[k]) << pp.sshift[k];
+        __syncthreads();  // the previous tile is no longer read
+        {
+            V2<R> in[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const uint64_t g = base | l2g | ((j & 1) ? t0 : 0) | ((j & 2) ? t1 : 0) | ((j & 4) ? t2 : 0);
+                in[j] = g < size ? psi[g] : mk<R>(0, 0);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; j++) tile[ft_slot<ES>(tid) ^ ft_slot<ES>(j * NTH)] = in[j];
+        }
+        __syncthreads();
+        double p[8];
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const uint32_t need = (pp.need >> (2 * g)) & 3u;
+            if (need == 0 && !(STRINGS && g == 3)) continue;
+            const int low = 3 * g, at = ft_slot<ES>(row[g]);
+            const int m0 = ft_slot<ES>(1 << low), m1 = ft_slot<ES>(2 << low), m2 = ft_slot<ES>(4 << low);
+            double2 v[8];
+#pragma unroll
+            for (int m = 0; m < 8; m++) {
+                const V2<R> x = tile[at ^ ((m & 1) ? m0 : 0) ^ ((m & 2) ? m1 : 0) ^ ((m & 4) ? m2 : 0)];
+                v[m] = make_double2((double)x.x, (double)x.y);
+            }
+            if (need & 1u) {
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+#pragma unroll
+                    for (int m = 0; m < 8; m++)
+                        if (!((m >> k) & 1)) re[g][k] = fma(v[m].x, v[m | (1 << k)].x, fma(v[m].y, v[m | (1 << k)].y, re[g][k]));
+            }
+            if (need & 2u) {  // -Im(x conj(y)): Y's sign
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+#pragma unroll
+                    for (int m = 0; m < 8; m++)
+                        if (!((m >> k) & 1)) im[g][k] = fma(v[m].x, v[m | (1 << k)].y, fma(-v[m].y, v[m | (1 << k)].x, im[g][k]));
+            }
+            if (STRINGS && g == 3) {
+#pragma unroll
+                for (int m = 0; m < 8; m++) p[m] = fma(v[m].x, v[m].x, v[m].y * v[m].y);
+            }
+        }
+        if constexpr (STRINGS) {
+            __syncthreads();  // the amplitudes are read
+            auto butterfly = [&] {
+#pragma unroll
+                for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+                    for (int m = 0; m < 8; m++)
+                        if (!(m & h)) {
+                            const double x = p[m], y = p[m | h];
+                            p[m] = x + y;
+                            p[m | h] = x - y;
+                        }
+            };
+            auto member = [&](int g, int m) {  // slot of member m of the thread's row of group g
+                return ft_slot<8>(row[g]) ^ ft_slot<8>(m << (3 * g));
+            };
+            butterfly();
+#pragma unroll
+            for (int m = 0; m < 8; m++) prob[member(3, m)] = p[m];
+#pragma unroll
+            for (int g = 2; g >= 0; g--) {
+                __syncthreads();
+#pragma unroll
+                for (int m = 0; m < 8; m++) p[m] = prob[member(g, m)];
+                butterfly();
+#pragma unroll
+                for (int m = 0; m < 8; m++) prob[member(g, m)] = p[m];
+            }
+            __syncthreads();
+            if (string) {
+                const double w = prob[ft_slot<8>(pp.zl[tid])];
+                az += (__popcll(base & pp.z[tid]) & 1) ? -w : w;
+            }
+        }
+    }
+    // columns: the threads' sums over wavefronts, then the wavefronts in index order; the strings as they are
+    __syncthreads();
+    double* red = reinterpret_cast<double*>(lds_raw);
+    const int lane = tid & 63, wave = tid >> 6;
+    constexpr int waves = NTH >> 6;
+#pragma unroll
+    for (int g = 0; g < 4; g++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const double x = wave_sum(re[g][k]), y = wave_sum(im[g][k]);
+            if (lane == 0) {
+                red[(2 * (3 * g + k)) * waves + wave] = x;
+                red[(2 * (3 * g + k) + 1) * waves + wave] = y;
+            }
+        }
+    __syncthreads();
+    if (tid < FT_COLS) {
+        double s = 0.0;
+        for (int x = 0; x < waves; x++) s += red[tid * waves + x];
+        partials[(uint64_t)tid * gridDim.x + blockIdx.x] = 2.0 * s;  // each pair stands for two amplitudes
+    }
+    if (string) partials[(uint64_t)(FT_COLS + tid) * gridDim.x + blockIdx.x] = az;
+}
+
+// term t's column of the passes' partials, summed into out[slot[t]]
+struct FColumns {
+    int16_t col[EXPECT_BATCH];
+    int32_t slot[EXPECT_BATCH];
+};
+__global__ void __launch_bounds__(RED_BLOCK) k_field_sums(const double* __restrict__ partials, unsigned cols,
+                                                          const FColumns fc, double* __restrict__ out) {
+    const double* col = partials + (uint64_t)fc.col[blockIdx.x] * cols;
+    double a = 0.0;
+    for (unsigned k = threadIdx.x; k < cols; k += blockDim.x) a += col[k];
+    a = block_sum(a);
+    if (threadIdx.x == 0) out[fc.slot[blockIdx.x]] = a;
+}
+
+// ------------------------------------------------------------------------------------------------
 static double finish_sum(State& s, double* partial, unsigned n) {
     double* out = partial + n;
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(RED_BLOCK), 0, s.stream, partial, (int)n, out);
@@ -381,10 +571,122 @@ static void queue_pauli_single(State& s, const PauliHost& t, double* partial, do
     QFVM_LAUNCHED();
 }
 
+// Z strings and single-qubit X / Y letters on the field kernel (see k_expect_fields). partials holds
+// EXPECT_PARTIALS doubles: a whole batch of strings and the flips of four passes on FT_GRID workgroups fit
+static void queue_fields(State& s, const PauliHost* terms, int n_terms, double* out_dev, double* partials, bool account) {
+    const int n = s.n;
+    constexpr int b = FT_BITS;
+    const int L = b < n ? (s.dtype == QFVM_C128 ? 3 : 4) : b;  // runs of 128 bytes
+    const uint64_t lowmask = (1ull << L) - 1;
+    const uint64_t tiles = b < n ? 1ull << (n - b) : 1;
+    // the partials of all passes wait for one summing launch: at most FT_COLS columns per pass and the strings
+    uint64_t high = 0;
+    int strings = 0;
+    for (int i = 0; i < n_terms; i++) {
+        high |= terms[i].flip & ~lowmask;
+        strings += terms[i].flip == 0;
+    }
+    const int per = b - L;
+    const int passes = std::max(1, per > 0 ? (__builtin_popcountll(high) + per - 1) / per : 1);
+    const unsigned fit = (unsigned)(EXPECT_PARTIALS / (size_t)(passes * FT_COLS + strings));
+    const unsigned grid = (unsigned)std::min<uint64_t>(tiles, std::min(FT_GRID, fit));
+    FColumns fc{};
+    int count = 0, done_cols = 0;
+    for (int ps = 0; ps < passes; ps++) {
+        uint64_t Qh = 0;
+        while (high && __builtin_popcountll(Qh) < per) {
+            Qh |= high & -high;
+            high &= high - 1;
+        }
+        const uint64_t asked = Qh | (ps == 0 ? lowmask : 0);  // flips taken in this pass
+        for (int q = L; q < n && __builtin_popcountll(Qh) < per; q++) Qh |= 1ull << q;
+        FPassArg pp{};
+        pp.size_bits = n;
+        int local_of[64];
+        for (int k = 0; k < 64; k++) local_of[k] = -1;
+        for (int q = 0, k = 0; k < b; q++)  // (qubits past the state pad small tiles)
+            if (q < L || q >= n || ((Qh >> q) & 1)) {
+                pp.q[k] = (uint8_t)q;
+                local_of[q] = k++;
+            }
+        for (int q = 0, k = 0, run = 0; q < n; q++) {  // the runs of qubits outside the tile; k: bit of its number
+            if (local_of[q] >= 0) continue;
+            if (k > 0 && local_of[q - 1] >= 0) run++;
+            pp.smask[run] |= 1u << k;
+            pp.sshift[run] = (uint32_t)(q - k);
+            k++;
+        }
+        const int classes = s.dtype == QFVM_C128 ? 3 : 4;
+        for (int g = 0; g < 4; g++) {
+            uint32_t used = 7u << (3 * g);
+            int k = 0;
+            for (int c = 0; c < classes; c++)  // lanes over one bit of each class: no bank conflicts
+                for (int l = 0; l < b; l++)
+                    if (l % classes == c && !((used >> l) & 1)) {
+                        used |= 1u << l;
+                        pp.row[g][k++] = (uint8_t)l;
+                        break;
+                    }
+            for (int l = 0; l < b; l++)
+                if (!((used >> l) & 1)) pp.row[g][k++] = (uint8_t)l;
+        }
+        for (int i = 0; i < n_terms; i++) {
+            const PauliHost& t = terms[i];
+            if (t.flip == 0) {
+                if (ps > 0) continue;
+                uint32_t zl = 0;
+                for (int k = 0; k < b; k++)
+                    if ((t.z >> pp.q[k]) & 1) zl |= 1u << k;
+                pp.z[pp.nz] = t.z;
+                pp.zl[pp.nz] = (uint16_t)zl;
+                fc.col[count] = (int16_t)(done_cols + FT_COLS + pp.nz++);
+            } else {
+                if (!(t.flip & asked)) continue;
+                const int k = local_of[t.flip_q];
+                pp.need |= (t.y ? 2u : 1u) << (2 * (k / 3));
+                fc.col[count] = (int16_t)(done_cols + 2 * k + (t.y ? 1 : 0));
+            }
+            fc.slot[count++] = t.slot;
+        }
+        std::optional<KernelScope> ks;
+        if (account) ks.emplace(s, "expect_tile", (double)s.size * s.amp_bytes());
+        double* to = partials + (size_t)done_cols * grid;
+        const size_t lds = ((size_t)1 << b) * std::max(s.amp_bytes(), sizeof(double));
+        auto launch = [&](auto kernel, auto* psi) {
+            hipLaunchKernelGGL(kernel, dim3(grid), dim3(FT_THREADS), lds, s.stream, psi, pp, tiles, to);
+        };
+        if (s.dtype == QFVM_C128) {
+            auto* psi = reinterpret_cast<const double2*>(s.psi);
+            pp.nz > 0 ? launch(k_expect_fields<double, true>, psi) : launch(k_expect_fields<double, false>, psi);
+        } else {
+            auto* psi = reinterpret_cast<const float2*>(s.psi);
+            pp.nz > 0 ? launch(k_expect_fields<float, true>, psi) : launch(k_expect_fields<float, false>, psi);
+        }
+        QFVM_LAUNCHED();
+        done_cols += FT_COLS + pp.nz;
+    }
+    std::optional<KernelScope> ks;  // its time is the reads' too
+    if (account) ks.emplace(s, "expect_tile", (double)done_cols * grid * sizeof(double));
+    hipLaunchKernelGGL(k_field_sums, dim3((unsigned)count), dim3(RED_BLOCK), 0, s.stream, partials, grid, fc, out_dev);
+    QFVM_LAUNCHED();
+}
+
 void queue_expectations(State& s, const PauliHost* terms, int n_terms, double* out_dev, double* partials,
                         double* fallback, bool account) {
     if (n_terms > EXPECT_BATCH) throw Error(QFVM_ERR_VALUE, "too many terms in one expectation batch");
     const int n = s.n;
+    // More than a few terms of one letter X or Y, or of Z letters only: the field kernel, whose cost does not
+    // grow with the terms and whose tiles hold more flip qubits. Short lists stay with one accumulator
+    // per term, which has less to do per tile (12 qubits: 12 terms 33 and 35 us, 24 terms 56 and 41 us; 24
+    // qubits at complex64: 8 Z terms 71 and 72 us, 12 terms 83 and 73 us), and a list with any other string
+    // stays there whole: its terms share the reads that the other strings need anyway.
+    bool fields = n_terms > (n >= 24 ? 8 : 12);
+    for (int i = 0; i < n_terms; i++)
+        fields = fields && (terms[i].flip == 0 || (terms[i].flip == (1ull << terms[i].flip_q) && (terms[i].z & ~terms[i].flip) == 0));
+    if (fields) {
+        queue_fields(s, terms, n_terms, out_dev, partials, account);
+        return;
+    }
     const int b = std::min(n, 11);  // 2^11 amplitudes per tile: 8 per thread (k_expect_tile<R, 8>)
     const int L = b < n ? std::min(5, b - 1) : b;
     const uint64_t lowmask = (1ull << L) - 1;
