@@ -257,6 +257,9 @@ void launch_zero(State& s, void* p, size_t bytes);  // bytes: a multiple of 8
 void allow_large_lds(const void* fn, int device);
 void launch_h2d_convert(State& s, const double* host, uint64_t n);  // host c128 -> device
 void launch_d2h_convert(State& s, double* host, uint64_t n);
+constexpr int POP_QUBITS = 14;
+// sums of |psi|^2 over the values of up to POP_QUBITS qubits (ascending; bit j of the index: qubits[j])
+void reduce_populations(State& s, const std::vector<int>& qubits, std::vector<double>& probs);
 double reduce_norm2(State& s);
 void reduce_probabilities(State& s, double* host_out);
 // Pauli-string expectations (expect_pauli's formula) of up to EXPECT_BATCH terms, queued on the

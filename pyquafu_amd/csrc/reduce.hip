@@ -1078,6 +1078,112 @@ double reduce_op_norm2(State& s, int q, const cd m[4]) {
 }
 
 // ------------------------------------------------------------------------------------------------
+// Joint populations of up to POP_QUBITS qubits: sum of |psi_i|^2 over the indices with each value of
+// the qubits' bits, for runs of noise channels. One read of the state, which bounds it from some 20 qubits;
+// below that a launch and the way to the host. The thread index is the low POP_LOW index bits, so
+// reads are whole lines whichever qubits are asked for; a workgroup has one value of the asked qubits
+// above them, and a slice of the other indices, so every bin's sum is built without atomics and in a
+// fixed order. With all qubits of a 14-qubit state asked it is one launch (timed with its caller, kraus_run).
+constexpr int POP_LOW = 8;
+struct PopArg {
+    uint32_t low;                    // asked qubits among the low POP_LOW
+    int nlow, nhigh;                 // numbers of asked qubits below and from POP_LOW on
+    int slice_bits;
+    uint64_t rest;                   // values of the other qubits from POP_LOW on
+    uint8_t high[POP_QUBITS];        // asked qubits from POP_LOW on
+    uint32_t smask[POP_QUBITS + 1], sshift[POP_QUBITS + 1];  // as in FPassArg, for the other qubits
+    int runs;
+};
+
+template <typename R>
+__global__ void __launch_bounds__(1 << POP_LOW) k_populations(const V2<R>* __restrict__ psi, uint64_t size, const PopArg a,
+                                                              double* __restrict__ out) {
+    __shared__ double sh[1 << POP_LOW];
+    const int tid = threadIdx.x;
+    const uint64_t slice = blockIdx.x & ((1u << a.slice_bits) - 1), hb = blockIdx.x >> a.slice_bits;
+    uint64_t base = tid;
+    for (int k = 0; k < a.nhigh; k++) base |= ((hb >> k) & 1ull) << a.high[k];
+    double acc = 0.0;
+    if (base < size) {
+#pragma unroll 4
+        for (uint64_t r = slice; r < a.rest; r += 1ull << a.slice_bits) {
+            uint64_t i = base;
+            for (int k = 0; k < a.runs; k++) i |= (r & a.smask[k]) << a.sshift[k];
+            const V2<R> v = psi[i];
+            acc = fma((double)v.x, (double)v.x, fma((double)v.y, (double)v.y, acc));
+        }
+    }
+    int bin = 0, at = 0;
+    bool writes = true;
+    for (int k = 0; k < POP_LOW; k++) {
+        if ((a.low >> k) & 1u) {
+            bin |= ((tid >> k) & 1) << at++;
+            continue;
+        }
+        writes = writes && !((tid >> k) & 1);
+        if (k < 6) {
+            acc += __shfl_xor(acc, 1 << k, 64);
+        } else {
+            sh[tid] = acc;
+            __syncthreads();
+            acc += sh[tid ^ (1 << k)];
+            __syncthreads();
+        }
+    }
+    if (writes) out[(((hb << a.nlow) | (uint64_t)bin) << a.slice_bits) | slice] = acc;
+}
+
+__global__ void __launch_bounds__(64) k_population_sums(const double* __restrict__ rows, int slice_bits,
+                                                        double* __restrict__ out) {
+    double acc = 0.0;
+    for (unsigned k = threadIdx.x; k < (1u << slice_bits); k += 64) acc += rows[((uint64_t)blockIdx.x << slice_bits) | k];
+    acc = wave_sum(acc);
+    if (threadIdx.x == 0) out[blockIdx.x] = acc;
+}
+
+// qubits ascending; bit j of probs' index is qubit qubits[j]. The last kernel writes to pinned memory.
+void reduce_populations(State& s, const std::vector<int>& qubits, std::vector<double>& probs) {
+    if (qubits.empty() || qubits.size() > (size_t)POP_QUBITS) throw Error(QFVM_ERR_VALUE, "too many qubits");
+    PopArg a{};
+    uint64_t asked = 0;
+    for (int q : qubits) {
+        asked |= 1ull << q;
+        if (q < POP_LOW)
+            a.nlow++;
+        else
+            a.high[a.nhigh++] = (uint8_t)q;
+    }
+    a.low = (uint32_t)(asked & ((1u << POP_LOW) - 1));
+    int rest = 0;
+    for (int q = POP_LOW; q < s.n; q++) {  // runs of the other qubits; rest: bit of their number
+        if ((asked >> q) & 1) continue;
+        if (rest == 0 || ((asked >> (q - 1)) & 1)) a.runs++;
+        a.smask[a.runs - 1] |= 1u << rest;
+        a.sshift[a.runs - 1] = (uint32_t)(q - rest);
+        rest++;
+    }
+    a.rest = 1ull << rest;
+    a.slice_bits = std::max(0, std::min(rest, 9 - a.nhigh));  // two workgroups per CU where the state has them
+    const size_t bins = (size_t)1 << qubits.size();
+    double* host = s.ensure_pinned(bins * sizeof(double));
+    double* rows = a.slice_bits ? reinterpret_cast<double*>(s.ensure_scratch((bins << a.slice_bits) * sizeof(double))) : host;
+    const dim3 grid(1u << (a.nhigh + a.slice_bits)), threads(1 << POP_LOW);
+    if (s.dtype == QFVM_C128)
+        hipLaunchKernelGGL(k_populations<double>, grid, threads, 0, s.stream, reinterpret_cast<const double2*>(s.psi),
+                           s.size, a, rows);
+    else
+        hipLaunchKernelGGL(k_populations<float>, grid, threads, 0, s.stream, reinterpret_cast<const float2*>(s.psi),
+                           s.size, a, rows);
+    QFVM_LAUNCHED();
+    if (a.slice_bits) {
+        hipLaunchKernelGGL(k_population_sums, dim3((unsigned)bins), dim3(64), 0, s.stream, rows, a.slice_bits, host);
+        QFVM_LAUNCHED();
+    }
+    QFVM_HIP(hipStreamSynchronize(s.stream));
+    probs.assign(host, host + bins);
+}
+
+// ------------------------------------------------------------------------------------------------
 // Amplitudes at given indices, and the overlap <a|b> of two states of one size (any dtypes).
 template <typename R>
 __global__ void k_gather(const V2<R>* __restrict__ psi, const uint64_t* __restrict__ idx, uint64_t n,
