@@ -307,6 +307,459 @@ __global__ void __launch_bounds__(256) k_seq_descend(const V2<R>* __restrict__ p
     out[s] = res;
 }
 
+// ------------------------------------------------------------------------------------------------
+// States of up to 4 GiB: every block end without a host round trip per binade.
+// The chunk loop above learns where S leaves a binade by reaching it, and waits for the host there: some
+// 25 times for 26 qubits. Here a first read sums the probabilities in any order. Such a sum A of the
+// blocks before b and the sequential S differ by their roundings, some sqrt(N) 2^-53 of S if these do not
+// conspire, so with a margin eps of 32 times that it tells the binade of every block but those whose
+// interval [A_b (1 - eps), A_b+1 (1 + eps)] holds a power of two. A second read forms the pairs of the former
+// (for their own binade) and marks the latter special: they are replayed with double additions, by one
+// thread, in order, each from the end of the one before and the composed pairs between. Blocks that cannot
+// change S (all p zero, or below half an ulp of both binades of the interval) are the identity and not
+// special. Exactness does not rest on the margin: every pair's use is checked against the exact S (its
+// binade, no carry out of it), and a check that fails, more than SEQ_SPECIALS special blocks, or sums that
+// are not finite send the call to the chunk loop.
+// What bounds it: two reads of the state, and some 40 us of launches up to 18 qubits; the chunk loop
+// reads once, so it stays the better one for larger states, whose reads outweigh its waits (SEQ_BYTES:
+// 28 qubits at complex128 1.84 -> 1.63 ms; two reads of 29 qubits would take 3.2, one and the waits 2.7).
+// Measured for one shot of a random complex128 state: 12 qubits 268 -> 48 us, 18 qubits 469 -> 52 us, 24
+// qubits 818 -> 151 us, 26 qubits 1.11 -> 0.45 ms.
+constexpr uint64_t SEQ_BYTES = 4ull << 30;
+constexpr unsigned SEQ_SPECIALS = 1024;
+constexpr int SEQ_IDENTITY = -32768;  // exponent entry of a block that keeps S
+constexpr double SEQ_TINY = 0x1p-1000;  // below it every block that changes S is special
+
+struct SegX {      // composed pairs since the last special block, and the number of special blocks
+    Xfer x;
+    unsigned count;
+};
+struct SeqSpecial {
+    uint64_t block;
+    Xfer before;  // pairs between the special block before and this one
+};
+struct SeqFast {
+    unsigned total;  // special blocks
+    int failed;
+};
+
+__device__ __forceinline__ SegX seg_compose(SegX f, SegX g) {
+    return SegX{g.count ? g.x : xcompose(f.x, g.x), f.count + g.count};
+}
+__device__ __forceinline__ SegX shfl_up_seg(SegX v, int off) {
+    return SegX{shfl_up_x(v.x, off), (unsigned)__shfl_up((int)v.count, off, 64)};
+}
+__device__ __forceinline__ SegX wave_scan_seg(SegX v, int lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const SegX o = shfl_up_seg(v, off);
+        if (lane >= off) v = seg_compose(o, v);
+    }
+    return v;
+}
+
+// sum of every tile's probabilities
+template <typename R>
+__global__ void __launch_bounds__(256) k_seq_mass(const V2<R>* __restrict__ psi, uint64_t size, double* __restrict__ mass,
+                                                  SeqFast* st) {
+    constexpr int TE = TILE_BLOCKS * SB;
+    __shared__ double wsum[4];
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0 && tid == 0) *st = SeqFast{0, 0};
+    const uint64_t at = (uint64_t)blockIdx.x * TE;
+    double a = 0.0;
+#pragma unroll
+    for (int r = 0; r < TE / 256; r++)
+        if (at + r * 256 + tid < size) a += prob_at<R>(psi, at + r * 256 + tid);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+    if ((tid & 63) == 0) wsum[tid >> 6] = a;
+    __syncthreads();
+    if (tid == 0) mass[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
+}
+
+// exclusive prefix sums of the tiles' masses; each workgroup of SCAN_GROUP tiles adds up those before its own
+__global__ void __launch_bounds__(SCAN_GROUP) k_seq_mass_prefix(const double* __restrict__ mass, uint64_t ntiles,
+                                                                double* __restrict__ pre) {
+    __shared__ double wtot[SCAN_GROUP / 64], wbefore[SCAN_GROUP / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const uint64_t first = (uint64_t)blockIdx.x * SCAN_GROUP;
+    double before = 0.0;
+#pragma unroll 8
+    for (uint64_t t = tid; t < first; t += SCAN_GROUP) before += mass[t];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
+    const double m = first + tid < ntiles ? mass[first + tid] : 0.0;
+    double inc = m;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const double o = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += o;
+    }
+    double ex = __shfl_up(inc, 1, 64);
+    if (lane == 0) {
+        ex = 0.0;
+        wbefore[wv] = before;
+    }
+    if (lane == 63) wtot[wv] = inc;
+    __syncthreads();
+    for (int j = 0; j < SCAN_GROUP / 64; j++) ex += wbefore[j] + (j < wv ? wtot[j] : 0.0);
+    if (first + tid < ntiles) pre[first + tid] = ex;
+}
+
+// Pairs of every block for its binade (bx, its exponent in be), the tile's special blocks (mask) and its
+// composition (tx). Threads as in k_seq_blocks.
+template <typename R>
+__global__ void __launch_bounds__(256) k_seq_pairs(const V2<R>* __restrict__ psi, uint64_t nblk,
+                                                   const double* __restrict__ pre, double eps, Xfer* __restrict__ bx,
+                                                   int16_t* __restrict__ be, uint64_t* __restrict__ mask,
+                                                   Xfer* __restrict__ tx, SeqFast* st) {
+    constexpr int TE = TILE_BLOCKS * SB, RUN = 8, ROWS = TE / 256;
+    __shared__ double pl[TE / RUN * (RUN + 1)];
+    __shared__ Xfer bl[TILE_BLOCKS];
+    __shared__ double wtot[4];
+    __shared__ uint64_t wmask[4];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    // (last tile first: the sums' read leaves the end of the state in the last-level cache)
+    const uint64_t tile = gridDim.x - 1 - blockIdx.x, tb0 = tile * TILE_BLOCKS;
+    const uint64_t ne = min((uint64_t)TILE_BLOCKS, nblk - tb0) * SB;
+    const V2<R>* __restrict__ src = psi + tb0 * SB;
+    {
+        double p[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const int e = r * 256 + tid;
+            p[r] = (uint64_t)e < ne ? prob_at<R>(src, e) : 0.0;
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const int e = r * 256 + tid;
+            pl[(e / RUN) * (RUN + 1) + e % RUN] = p[r];
+        }
+    }
+    __syncthreads();
+    double p[RUN], q = 0.0, most = 0.0;
+#pragma unroll
+    for (int j = 0; j < RUN; j++) {
+        p[j] = pl[tid * (RUN + 1) + j];
+        q += p[j];
+        most = fmax(most, p[j]);
+    }
+#pragma unroll
+    for (int o = 1; o < SB / RUN; o <<= 1) {  // over the block's four threads
+        q += __shfl_xor(q, o, 64);
+        most = fmax(most, __shfl_xor(most, o, 64));
+    }
+    double inc = q;  // over the wavefront's 16 blocks
+#pragma unroll
+    for (int off = SB / RUN; off < 64; off <<= 1) {
+        const double o = __shfl_up(inc, off, 64);
+        if (lane >= off) inc += o;
+    }
+    if (lane == 63) wtot[wv] = inc;
+    __syncthreads();
+    double a0 = pre[tile] + (inc - q);
+    for (int j = 0; j < wv; j++) a0 += wtot[j];
+    const double a1 = a0 + q;
+    const double lo = a0 * (1.0 - eps), hi = a1 * (1.0 + eps);
+    bool special = false;
+    int e = SEQ_IDENTITY;
+    if (!(a1 <= 1.7976931348623157e308)) {
+        st->failed = 1;
+    } else if (q > 0.0) {
+        if (lo < SEQ_TINY) {
+            special = true;
+        } else {
+            e = ilogb(lo);
+            const int eh = ilogb(hi);
+            if (eh > e) {
+                special = eh > e + 1 || !(most < ldexp(1.0, e - 53));
+                e = SEQ_IDENTITY;
+            }
+        }
+    }
+    // Without a tie the pair's entries are equal, the sum of the rounded steps: whole numbers below 2^53 (the
+    // block ends below its binade's top), exact in double.
+    Xfer x{0, 0};
+    double sum = 0.0;
+    bool tie = false;
+    if (e != SEQ_IDENTITY) {
+#pragma unroll
+        for (int j = 0; j < RUN; j++) {
+            const double f = ldexp(p[j], 52 - e), w = rint(f);
+            tie = tie || fabs(f - w) == 0.5;
+            sum += w;
+        }
+    }
+    if (__any(tie)) {
+        if (e != SEQ_IDENTITY) {
+            const double lim = ldexp(1.0, e + 1);
+            for (int j = 0; j < RUN; j++) x = xcompose(x, xelem(pl[tid * (RUN + 1) + j], 52 - e, lim));
+        }
+        x = lane_tree_x(x, lane, SB / RUN);
+    } else {
+#pragma unroll
+        for (int o = 1; o < SB / RUN; o <<= 1) sum += __shfl_xor(sum, o, 64);
+        x.w0 = x.w1 = (int64_t)sum;
+    }
+    uint64_t marks = __ballot(special && (lane & (SB / RUN - 1)) == 0);  // bits 0, 4, 8, ...: to bits 0, 1, 2, ...
+    if ((tid & (SB / RUN - 1)) == 0) {
+        const int b = tid / (SB / RUN);
+        bl[b] = x;
+        if (tb0 + b < nblk) {
+            bx[tb0 + b] = x;
+            be[tb0 + b] = (int16_t)e;
+        }
+    }
+    if (lane == 0) {
+        uint64_t m = 0;
+        for (int b = 0; b < 16; b++) m |= ((marks >> (4 * b)) & 1ull) << b;
+        wmask[wv] = m;
+    }
+    __syncthreads();
+    if (tid < TILE_BLOCKS) {
+        const uint64_t m = wmask[0] | (wmask[1] << 16) | (wmask[2] << 32) | (wmask[3] << 48);
+        // pairs after the last special block (all, if there is none)
+        const bool counts = m == 0 || tid > 63 - __clzll((long long)m);
+        const Xfer t = lane_tree_x(counts ? bl[tid] : Xfer{0, 0}, tid, TILE_BLOCKS);
+        if (tid == 0) {
+            tx[tile] = t;
+            mask[tile] = m;
+        }
+    }
+}
+
+__device__ __forceinline__ SegX seg_tile(const Xfer* __restrict__ tx, const uint64_t* __restrict__ mask, uint64_t t,
+                                         uint64_t ntiles) {
+    return t < ntiles ? SegX{tx[t], (unsigned)__popcll(mask[t])} : SegX{Xfer{0, 0}, 0};
+}
+
+// composition of each group of SCAN_GROUP consecutive tiles
+__global__ void __launch_bounds__(SCAN_GROUP) k_seg_group_sums(const Xfer* __restrict__ tx,
+                                                               const uint64_t* __restrict__ mask, uint64_t ntiles,
+                                                               SegX* __restrict__ gx) {
+    __shared__ SegX wt[SCAN_GROUP / 64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const SegX v = wave_scan_seg(seg_tile(tx, mask, (uint64_t)blockIdx.x * SCAN_GROUP + tid, ntiles), lane);
+    if (lane == 63) wt[tid >> 6] = v;
+    __syncthreads();
+    if (tid == 0) {
+        SegX g = wt[0];
+        for (int j = 1; j < SCAN_GROUP / 64; j++) g = seg_compose(g, wt[j]);
+        gx[blockIdx.x] = g;
+    }
+}
+
+// exclusive prefix of every tile (as k_seq_tile_prefix); the last one's inclusive count is the total
+__global__ void __launch_bounds__(SCAN_GROUP) k_seg_tile_prefix(const Xfer* __restrict__ tx,
+                                                                const uint64_t* __restrict__ mask, uint64_t ntiles,
+                                                                const SegX* __restrict__ gx, SegX* __restrict__ tpre,
+                                                                SeqFast* st) {
+    __shared__ SegX wt[SCAN_GROUP / 64];
+    __shared__ SegX gpre;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const uint64_t g = blockIdx.x;
+    if (wv == 0) {
+        const uint64_t per = (g + 63) / 64;
+        const uint64_t a = (uint64_t)lane * per, b = min(a + per, g);
+        SegX x{Xfer{0, 0}, 0};
+        for (uint64_t i = a; i < b; i++) x = seg_compose(x, gx[i]);
+        x = wave_scan_seg(x, lane);
+        if (lane == 63) gpre = x;
+    }
+    const uint64_t t = g * SCAN_GROUP + tid;
+    const SegX inc = wave_scan_seg(seg_tile(tx, mask, t, ntiles), lane);
+    SegX ex = shfl_up_seg(inc, 1);
+    if (lane == 0) ex = SegX{Xfer{0, 0}, 0};
+    if (lane == 63) wt[wv] = inc;
+    __syncthreads();
+    SegX pre = gpre;
+    for (int j = 0; j < wv; j++) pre = seg_compose(pre, wt[j]);
+    if (t < ntiles) tpre[t] = seg_compose(pre, ex);
+    if (t == ntiles - 1) st->total = pre.count + inc.count;
+}
+
+// block `lane` of tile t: the pairs since the last special block, its own included (identity for a special one)
+__device__ __forceinline__ Xfer seg_block(const Xfer* __restrict__ bx, const SegX& pre, uint64_t m, uint64_t t, int lane,
+                                          uint64_t nblk) {
+    const uint64_t cb = t * TILE_BLOCKS + lane;
+    const SegX v{cb < nblk ? bx[cb] : Xfer{0, 0}, (unsigned)((m >> lane) & 1ull)};
+    const SegX inc = wave_scan_seg(v, lane);
+    return inc.count ? inc.x : xcompose(pre.x, inc.x);
+}
+
+// the special blocks in order, one wavefront per tile
+__global__ void __launch_bounds__(256) k_seq_specials(const Xfer* __restrict__ bx, const uint64_t* __restrict__ mask,
+                                                      const SegX* __restrict__ tpre, uint64_t ntiles, uint64_t nblk,
+                                                      SeqSpecial* __restrict__ sp) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t t = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= ntiles) return;  // whole wavefronts
+    const uint64_t m = mask[t];
+    if (m == 0) return;
+    const SegX pre = tpre[t];
+    const Xfer x = seg_block(bx, pre, m, t, lane, nblk);
+    Xfer before = shfl_up_x(x, 1);
+    if (lane == 0) before = pre.x;
+    const unsigned k = pre.count + (unsigned)__popcll(m & ((1ull << lane) - 1));
+    if (((m >> lane) & 1ull) && k < SEQ_SPECIALS) sp[k] = SeqSpecial{t * TILE_BLOCKS + lane, before};
+}
+
+// m 2^(e-52) for the S that the pairs x make of s (s itself where they change nothing)
+__device__ __forceinline__ double seq_after(double s, Xfer x, int* e, int64_t* m) {
+    *e = ilogb(s);
+    const int64_t m0 = (int64_t)ldexp(s, 52 - *e);
+    const int64_t w = (m0 & 1) ? x.w1 : x.w0;
+    *m = m0 + w;
+    return w ? ldexp((double)*m, *e - 52) : s;
+}
+
+// S at the end of every special block: their probabilities are staged in LDS, then one thread adds in order
+template <typename R>
+__global__ void __launch_bounds__(256) k_seq_resolve(const V2<R>* __restrict__ psi, const SeqSpecial* __restrict__ sp,
+                                                     double* __restrict__ ends, SeqFast* st) {
+    constexpr int BATCH = 128;
+    __shared__ double p[BATCH * SB];
+    __shared__ Xfer before[BATCH];
+    const unsigned total = st->total;
+    if (total > SEQ_SPECIALS) {
+        if (threadIdx.x == 0) st->failed = 1;
+        return;
+    }
+    double s = 0.0;
+    for (unsigned k0 = 0; k0 < total; k0 += BATCH) {
+        const unsigned n = min((unsigned)BATCH, total - k0);
+        __syncthreads();
+        for (unsigned i = threadIdx.x; i < n * SB; i += 256) p[i] = prob_at<R>(psi, sp[k0 + i / SB].block * SB + i % SB);
+        for (unsigned i = threadIdx.x; i < n; i += 256) before[i] = sp[k0 + i].before;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (unsigned k = 0; k < n; k++) {
+                int e;
+                int64_t m;
+                if (s > 0.0) s = seq_after(s, before[k], &e, &m);
+#pragma unroll
+                for (int j = 0; j < SB; j++) s = __dadd_rn(s, p[k * SB + j]);
+                ends[k0 + k] = s;
+            }
+    }
+}
+
+// S at every block end, and the check of every pair's binade
+__global__ void __launch_bounds__(256) k_seq_ends(const Xfer* __restrict__ bx, const int16_t* __restrict__ be,
+                                                  const uint64_t* __restrict__ mask, const SegX* __restrict__ tpre,
+                                                  uint64_t ntiles, uint64_t nblk, const double* __restrict__ ends,
+                                                  double* __restrict__ B, SeqFast* st) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t t = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= ntiles || st->total > SEQ_SPECIALS) return;
+    const uint64_t m = mask[t];
+    const SegX pre = tpre[t];
+    const Xfer x = seg_block(bx, pre, m, t, lane, nblk);
+    const uint64_t cb = t * TILE_BLOCKS + lane;
+    if (cb >= nblk) return;
+    const unsigned k = pre.count + (unsigned)__popcll(m & ((2ull << lane) - 1));  // special blocks up to this one
+    const double s = k > 0 ? ends[k - 1] : 0.0;
+    const int want = be[cb];
+    double end = s;
+    bool good = s <= 1.7976931348623157e308;
+    if (s > 0.0 && good) {
+        int e;
+        int64_t mm;
+        end = seq_after(s, x, &e, &mm);
+        if (want != SEQ_IDENTITY) good = want == e && mm < M_CROSS;
+    } else if (want != SEQ_IDENTITY) {
+        good = false;
+    }
+    if (!good) st->failed = 1;
+    B[cb] = end;
+}
+
+
+// Block ends and shots of a state of up to SEQ_BYTES. False: nothing was written, the chunk loop has to run.
+template <typename R>
+static bool sample_fast(State& s, const double* host_u, int64_t shots, uint64_t* host_out) {
+    const uint64_t nblk = s.size / SB;
+    const uint64_t ntiles = (nblk + TILE_BLOCKS - 1) / TILE_BLOCKS;
+    const uint64_t ngroups = (ntiles + SCAN_GROUP - 1) / SCAN_GROUP;
+    size_t bytes = 0;
+    auto part = [&](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) & ~size_t(255);
+        return at;
+    };
+    const size_t oB = part(nblk * sizeof(double)), obx = part(nblk * sizeof(Xfer)), obe = part(nblk * sizeof(int16_t));
+    const size_t omass = part(ntiles * sizeof(double)), opre = part(ntiles * sizeof(double)), omask = part(ntiles * sizeof(uint64_t));
+    const size_t otx = part(ntiles * sizeof(Xfer)), otpre = part(ntiles * sizeof(SegX)), ogx = part(ngroups * sizeof(SegX));
+    const size_t osp = part(SEQ_SPECIALS * sizeof(SeqSpecial)), oends = part(SEQ_SPECIALS * sizeof(double));
+    const size_t ost = part(sizeof(SeqFast));
+    // a few shots: their uniforms and results stay in pinned memory, which the search reads and writes
+    const bool few = shots <= 1024;
+    const size_t ou = part(few ? 0 : (size_t)shots * sizeof(double)), oo = part(few ? 0 : (size_t)shots * sizeof(uint64_t));
+    char* base = reinterpret_cast<char*>(s.ensure_scratch(bytes));
+    const size_t per = few ? (size_t)shots : 0;
+    double* pin = s.ensure_pinned(sizeof(SeqFast) + per * (sizeof(double) + sizeof(uint64_t)));
+    SeqFast* hst = reinterpret_cast<SeqFast*>(pin);
+    static_assert(sizeof(SeqFast) == sizeof(double), "pinned layout");
+    double* hu = pin + 1;
+    uint64_t* ho = reinterpret_cast<uint64_t*>(hu + per);
+    auto at = [&](size_t o) { return base + o; };
+    double* B = reinterpret_cast<double*>(at(oB));
+    Xfer *bx = reinterpret_cast<Xfer*>(at(obx)), *tx = reinterpret_cast<Xfer*>(at(otx));
+    int16_t* be = reinterpret_cast<int16_t*>(at(obe));
+    double *mass = reinterpret_cast<double*>(at(omass)), *pre = reinterpret_cast<double*>(at(opre)), *ends = reinterpret_cast<double*>(at(oends));
+    uint64_t* mask = reinterpret_cast<uint64_t*>(at(omask));
+    SegX *tpre = reinterpret_cast<SegX*>(at(otpre)), *gx = reinterpret_cast<SegX*>(at(ogx));
+    SeqSpecial* sp = reinterpret_cast<SeqSpecial*>(at(osp));
+    SeqFast* st = reinterpret_cast<SeqFast*>(at(ost));
+    double* du = few ? hu : reinterpret_cast<double*>(at(ou));
+    uint64_t* dout = few ? ho : reinterpret_cast<uint64_t*>(at(oo));
+    const V2<R>* psi = reinterpret_cast<const V2<R>*>(s.psi);
+    const double eps = (32.0 * std::sqrt((double)s.size) + 1024.0) * 0x1p-53;
+    const dim3 tiles((unsigned)ntiles), waves((unsigned)((ntiles + 3) / 4)), groups((unsigned)ngroups);
+    if (few)
+        std::copy(host_u, host_u + shots, hu);
+    else
+        QFVM_HIP(hipMemcpyAsync(du, host_u, (size_t)shots * sizeof(double), hipMemcpyHostToDevice, s.stream));
+    {
+        KernelScope ks(s, "sample_scan", 2.0 * (double)s.size * s.amp_bytes() + (double)nblk * sizeof(double));
+        hipLaunchKernelGGL(k_seq_mass<R>, tiles, dim3(256), 0, s.stream, psi, s.size, mass, st);
+        QFVM_LAUNCHED();
+        hipLaunchKernelGGL(k_seq_mass_prefix, groups, dim3(SCAN_GROUP), 0, s.stream, mass, ntiles, pre);
+        QFVM_LAUNCHED();
+        hipLaunchKernelGGL(k_seq_pairs<R>, tiles, dim3(256), 0, s.stream, psi, nblk, pre, eps, bx, be, mask, tx, st);
+        QFVM_LAUNCHED();
+        if (ngroups > 1) {
+            hipLaunchKernelGGL(k_seg_group_sums, groups, dim3(SCAN_GROUP), 0, s.stream, tx, mask, ntiles, gx);
+            QFVM_LAUNCHED();
+        }
+        hipLaunchKernelGGL(k_seg_tile_prefix, groups, dim3(SCAN_GROUP), 0, s.stream, tx, mask, ntiles, gx, tpre, st);
+        QFVM_LAUNCHED();
+        hipLaunchKernelGGL(k_seq_specials, waves, dim3(256), 0, s.stream, bx, mask, tpre, ntiles, nblk, sp);
+        QFVM_LAUNCHED();
+        hipLaunchKernelGGL(k_seq_resolve<R>, dim3(1), dim3(256), 0, s.stream, psi, sp, ends, st);
+        QFVM_LAUNCHED();
+        hipLaunchKernelGGL(k_seq_ends, waves, dim3(256), 0, s.stream, bx, be, mask, tpre, ntiles, nblk, ends, B, st);
+        QFVM_LAUNCHED();
+    }
+    {
+        KernelScope ks(s, "sample_search", (double)shots * (8.0 + SB * (double)s.amp_bytes()));
+        hipLaunchKernelGGL(k_seq_descend<R>, dim3((unsigned)((shots + 255) / 256)), dim3(256), 0, s.stream, psi, B, nblk,
+                           SB, s.n, du, shots, dout);
+        QFVM_LAUNCHED();
+    }
+    QFVM_HIP(hipMemcpyAsync(hst, st, sizeof(SeqFast), hipMemcpyDeviceToHost, s.stream));
+    QFVM_HIP(hipStreamSynchronize(s.stream));
+    if (hst->failed) return false;
+    if (few)
+        std::copy(ho, ho + shots, host_out);
+    else {
+        QFVM_HIP(hipMemcpyAsync(host_out, dout, (size_t)shots * sizeof(uint64_t), hipMemcpyDeviceToHost, s.stream));
+        QFVM_HIP(hipStreamSynchronize(s.stream));
+    }
+    return true;
+}
+
 template <typename R>
 static void sample_typed(State& s, const double* host_u, int64_t shots, uint64_t* host_out) {
     const int n = s.n;
@@ -428,6 +881,10 @@ static void sample_typed(State& s, const double* host_u, int64_t shots, uint64_t
 
 void sample_sequential_rule(State& s, const double* host_u, int64_t shots, uint64_t* host_out) {
     if (shots <= 0) return;
+    if (s.size >= (uint64_t)SB && (uint64_t)s.size * s.amp_bytes() <= SEQ_BYTES &&
+        (s.dtype == QFVM_C128 ? sample_fast<double>(s, host_u, shots, host_out)
+                              : sample_fast<float>(s, host_u, shots, host_out)))
+        return;
     if (s.dtype == QFVM_C128)
         sample_typed<double>(s, host_u, shots, host_out);
     else
