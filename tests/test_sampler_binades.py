@@ -59,8 +59,8 @@ def test_block_ends_of_groups(n, kind):
     _check(n, kind, "c128", 20000)
 
 
-# up to 1024 shots stay in pinned memory
-@pytest.mark.parametrize("shots", [1, 2, 1024, 1025])
+# up to 2^20 shots stay in pinned memory
+@pytest.mark.parametrize("shots", [1, 2, 1024, 1 << 20, (1 << 20) + 1])
 def test_shot_counts(shots):
     _check(13, "random", "c128", shots)
 
