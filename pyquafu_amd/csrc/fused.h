@@ -114,9 +114,11 @@ inline int mat_ext(int b) { return b - 8 < MAT_MAX_EXT ? b - 8 : MAT_MAX_EXT; }
 // tiles in LDS). complex128: 2^11-amplitude tiles, which let four workgroups share a CU (faster than
 // 2^12 at 24 to 33 qubits by 1.5 to 3 %); complex64: 2^12 (one state: 41% of HBM peak per 30-qubit
 // pass against 39% at 2^13, 33-qubit QFT 234 vs 249 ms). Contiguous runs of 32 amplitudes for one
-// state and 64 for two.
+// state; for two, 64 at complex64 and 8 (whole lines) at complex128, which leaves 8 chosen qubits: 24
+// qubits, 8 layers of rotations and a CZ ring take 10 reverse passes instead of 15 (16.1 -> 12.1 ms with
+// fuller gradient stages; 26 qubits 61 -> 54).
 inline int default_tile_bits(int dtype, int /*states*/) { return dtype == QFVM_C128 ? 11 : 12; }
-inline int default_low_bits(int /*dtype*/, int states) { return states == 1 ? 5 : 6; }
+inline int default_low_bits(int dtype, int states) { return states == 1 ? 5 : dtype == QFVM_C128 ? 3 : 6; }
 
 // One item of an execution plan: a fused pass or a single gate for the per-gate kernels.
 struct PlanItem {

@@ -397,61 +397,163 @@ __device__ void grad_stage(const V2<R>* phi, const V2<R>* lam, int T, uint64_t g
     }
 }
 
+// a DPP move of both halves; every lane of the wavefront must be active
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// a's total over lane pairs ROWS apart in the lanes without that bit, b's in those with it: the swap
+// instructions exchange a's upper rows with b's lower ones
+template <int ROWS>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    const uint64_t ua = __builtin_bit_cast(uint64_t, a), ub = __builtin_bit_cast(uint64_t, b);
+    auto swap = [](uint32_t x, uint32_t y) {
+        if constexpr (ROWS == 32)
+            return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        else
+            return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    };
+    const auto lo = swap((uint32_t)ua, (uint32_t)ub), hi = swap((uint32_t)(ua >> 32), (uint32_t)(ub >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((uint64_t)hi[1] << 32) | lo[1]);
+}
+
 // Sum over the wavefront of 8 values at once: a transposing butterfly (each exchange halves the
-// values a lane keeps) takes 10 double shuffles instead of 8 x 6. Returns, in every lane, the
-// total of value m = 4 * lane bit 5 + 2 * lane bit 4 + lane bit 3.
+// values a lane keeps) without a select or an LDS permute: lane swaps, then DPP moves. Returns, in every
+// lane, the total of value m = 4 * lane bit 5 + 2 * lane bit 4 + lane bit 3.
 __device__ __forceinline__ double wave_total8(const double (&a)[8], int lane) {
-    const bool b5 = (lane >> 5) & 1, b4 = (lane >> 4) & 1, b3 = (lane >> 3) & 1;
     double t4[4], t2[2];
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const double keep = b5 ? a[k + 4] : a[k], give = b5 ? a[k] : a[k + 4];
-        t4[k] = keep + __shfl_xor(give, 32, 64);
-    }
+    for (int k = 0; k < 4; k++) t4[k] = swap_add<32>(a[k], a[k + 4]);
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-        const double keep = b4 ? t4[k + 2] : t4[k], give = b4 ? t4[k] : t4[k + 2];
-        t2[k] = keep + __shfl_xor(give, 16, 64);
-    }
-    double t = (b3 ? t2[1] : t2[0]) + __shfl_xor(b3 ? t2[0] : t2[1], 8, 64);
-    t += __shfl_xor(t, 4, 64);
-    t += __shfl_xor(t, 2, 64);
-    t += __shfl_xor(t, 1, 64);
+    for (int k = 0; k < 2; k++) t2[k] = swap_add<16>(t4[k], t4[k + 2]);
+    const bool b3 = (lane >> 3) & 1;
+    double t = (b3 ? t2[1] : t2[0]) + dpp_move<0x128>(b3 ? t2[0] : t2[1]);  // row_ror:8
+    t += dpp_move<0x141>(t);                                                // row_half_mirror
+    t += dpp_move<0xB1>(t);                                                 // quad_perm [1, 0, 3, 2]
+    t += dpp_move<0x4E>(t);                                                 // quad_perm [2, 3, 0, 1]
     return t;
 }
 
-// grad_stage for the split-row kernel, whose threads hold exactly 8 elements each (NT = T / 8):
-// element j of thread tid is j * NT + tid, its global index g_tid | pd.top[j] (no per-element
-// index walk). Im(conj(lam) phi) of the elements is computed once per stage and kept in registers
-// across the markers (Z markers read nothing more), and the wavefront sums of 8 markers take one
-// transposing butterfly. Same partial sums as grad_stage: the same per-thread order over
-// elements, the same exchange partners over the wavefront, the same order over wavefronts.
+// Gradient markers of a stage in the split-row kernel, whose threads hold exactly 8 elements each (NT =
+// T / 8). Uncontrolled markers share what they read: the sums that they can need are taken at once, and a
+// marker picks its own.
+//   * X and Y on tile bits (complex128): the bits fall into four groups of three (the last one the top three);
+//     a thread gathers the 8 members of a group from both tiles and adds up the products with each member's
+//     partner over each bit asked for: 16 reads for up to six markers, where each took 16. At complex64 the
+//     members as doubles do not fit the 128 registers that its 512 threads leave (24 qubits: 7.03 -> 7.65
+//     ms with it), so those markers read on their own, as the controlled ones do.
+//   * Z: a thread's sum of w = Im(conj(lam) phi) over its elements (element j of thread tid is j * NT + tid),
+//     and that sum signed by each of the top three bits and by each of its six lane bits; other tile
+//     bits are the wavefront's number, qubits outside the tile sign the whole.
+// Which sums a stage needs and where each marker finds its own comes with the op records (grad_info): a loop
+// over the records here is a chain of scalar loads that costs more than the sums.
+// Bound by the LDS reads. 24 qubits, 8 layers of 48 markers, reverse sweep at complex128 13.4 -> 12.3 ms
+// with it before grad_info and the wider runs of chosen qubits (default_low_bits), 9.5 ms with both; at
+// complex64 7.03 -> 6.65 ms.
+// red: GRAD_RED doubles, column c of wavefront w at c * 8 + w: 8 g + 3 y + k the group sums, 32 the whole, 33
+// to 35 the top bits, 36 to 41 the lane bits; controlled markers use it afterwards, 8 at a time.
+constexpr int GRAD_RED = 42 * 8;
 template <typename R>
 __device__ void grad_stage8(const V2<R>* phi, const V2<R>* lam, uint64_t g_tid, const PassDesc& pd,
                             const FOpDev<R>* __restrict__ ops, int cnt, double* red, double* __restrict__ partials,
                             uint64_t tiles) {
-    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6, waves = NT >> 6, b = pd.b;
+    const int total8_of = (((lane >> 5) & 1) << 2) | (((lane >> 4) & 1) << 1) | ((lane >> 3) & 1);
+    const uint64_t info = ops[0].pxmask;  // of the stage (grad_info)
+    const uint32_t need = (uint32_t)info;
+    const int alone = (int)((info >> 32) & 0xffffu);  // markers on their own, which come first
+    const bool z = (info >> 48) & 1u;
+    for (int g = 0; g < 4; g++) {
+        if (sizeof(R) == 4) break;
+        const uint32_t cols = (need >> (8 * g)) & 63u;
+        if (cols == 0) continue;
+        const int lo = g < 3 ? 3 * g : b - 3;
+        // the rows of the lowest group are dealt to the lanes by bits 4, 5, 6, 3, ...: no bank conflicts
+        const int row = lo == 0 ? ((tid & 7) << 4) | (tid & 8) | ((tid >> 4) << 7)
+                                : ((tid >> lo) << (lo + 3)) | (tid & ((1 << lo) - 1));
+        const int at = swz(row), o0 = swz(1 << lo), o1 = swz(2 << lo), o2 = swz(4 << lo);
+        V2<R> v[8], u[8];
+#pragma unroll
+        for (int m = 0; m < 8; m++) {
+            const int e = at ^ ((m & 1) ? o0 : 0) ^ ((m & 2) ? o1 : 0) ^ ((m & 4) ? o2 : 0);
+            v[m] = phi[e];
+            u[m] = lam[e];
+        }
+        double acc[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc[k] = 0.0;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if ((cols >> k) & 1u) {
+                double a = 0.0;
+#pragma unroll
+                for (int m = 0; m < 8; m++) {
+                    const V2<R> q = v[m ^ (1 << k)];
+                    a = fma((double)u[m].x, (double)q.y, fma(-(double)u[m].y, (double)q.x, a));
+                }
+                acc[k] = a;
+            }
+            if ((cols >> (3 + k)) & 1u) {  // (Y psi)[e] = +i q where the bit of e is set, -i q where clear
+                double a = 0.0;
+#pragma unroll
+                for (int m = 0; m < 8; m++) {
+                    const V2<R> q = v[m ^ (1 << k)];
+                    const double s = ((m >> k) & 1) ? 1.0 : -1.0;
+                    a = fma(s * (double)u[m].x, (double)q.x, fma(s * (double)u[m].y, (double)q.y, a));
+                }
+                acc[3 + k] = a;
+            }
+        }
+        const double t = wave_total8(acc, lane);
+        if ((lane & 7) == 0) red[(8 * g + total8_of) * 8 + wave] = t;
+    }
     double w[8];  // Im(conj(lam) phi) of the thread's elements
+    if (z || alone) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int e = j * NT + tid;
-        const V2<R> p = phi[swz(e)], l = lam[swz(e)];
-        w[j] = (double)l.x * p.y - (double)l.y * p.x;
+        for (int j = 0; j < 8; j++) {
+            const int e = j * NT + tid;
+            const V2<R> p = phi[swz(e)], l = lam[swz(e)];
+            w[j] = (double)l.x * p.y - (double)l.y * p.x;
+        }
     }
-    // An uncontrolled Z marker's sum over the thread's elements, in the element order of the
-    // general loop below (so the same roundings): on one of the tile's three top bits (bit kk of
-    // the element number j), wt[kk] = sum of (bit kk of j ? -w : w); on any other qubit the sign is
-    // the lane's own index bit, the same for all 8 elements: +-wsum.
-    double wsum = 0.0, wt[3] = {0.0, 0.0, 0.0};
+    if (z) {
+        double acc[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        wsum += w[j];
+        for (int k = 0; k < 8; k++) acc[k] = 0.0;
 #pragma unroll
-        for (int kk = 0; kk < 3; kk++) wt[kk] += ((j >> kk) & 1) ? -w[j] : w[j];
+        for (int j = 0; j < 8; j++) {
+            acc[0] += w[j];
+#pragma unroll
+            for (int kk = 0; kk < 3; kk++) acc[1 + kk] += ((j >> kk) & 1) ? -w[j] : w[j];
+        }
+        const double wsum = acc[0];
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[4 + k] = ((lane >> k) & 1) ? -wsum : wsum;
+        double t = wave_total8(acc, lane);
+        if ((lane & 7) == 0) red[(32 + total8_of) * 8 + wave] = t;
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc[k] = k < 2 ? (((lane >> (4 + k)) & 1) ? -wsum : wsum) : 0.0;
+        t = wave_total8(acc, lane);
+        if ((lane & 7) == 0 && total8_of < 2) red[(40 + total8_of) * 8 + wave] = t;
     }
-    const int top0 = pd.q[pd.b - 3], top1 = pd.q[pd.b - 2], top2 = pd.q[pd.b - 1];
-    for (int c0 = 0; c0 < cnt; c0 += 8) {
-        const int cn = min(8, cnt - c0);
+    __syncthreads();
+    for (int c = alone + tid; c < cnt; c += NT) {
+        const FOpDev<R>& o = ops[c];
+        const uint32_t at = (uint32_t)(o.pxmask >> 49);  // of the marker (grad_info)
+        const int col = at & 63, flips = (at >> 6) & 7;  // flips: wavefronts whose sums change sign
+        const bool neg = ((at >> 9) & 1u) && ((g_tid >> o.cm_group) & 1ull);
+        double sum = 0.0;
+        for (int wv = 0; wv < waves; wv++) sum += (wv & flips) ? -red[col * 8 + wv] : red[col * 8 + wv];
+        partials[(uint64_t)o.flags * tiles + blockIdx.x] = neg ? -sum : sum;
+    }
+    __syncthreads();
+    for (int c0 = 0; c0 < alone; c0 += 8) {
+        const int cn = min(8, alone - c0);
         double acc[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) acc[k] = 0.0;
@@ -463,65 +565,85 @@ __device__ void grad_stage8(const V2<R>* phi, const V2<R>* lam, uint64_t g_tid, 
             uint64_t gk = g_tid;
             asm volatile("" : "+v"(tk), "+v"(gk));
             double a = 0.0;
-            if (o.g == GEN_Z && o.cm_ext == 0) {
-                const int q = (int)o.cm_group;
-                a = q == top0 ? wt[0]
-                    : q == top1 ? wt[1]
-                    : q == top2 ? wt[2]
-                    : (((gk >> q) & 1ull) ? 0.0 - wsum : wsum);  // 0 - x: +0 for x = +0, as the loop gives
-            } else if (o.g == GEN_Z) {
+            if (o.g == GEN_Z) {
 #pragma unroll
                 for (int j = 0; j < 8; j++) {
                     const uint64_t gi = gk | pd.top[j];
                     const double v = ((gi >> o.cm_group) & 1ull) ? -w[j] : w[j];
                     a += ((gi & o.cm_ext) == o.cm_ext) ? v : 0.0;
                 }
-            } else if (o.cm_ext == 0) {  // uncontrolled X / Y: no index tests
-                const int lb = (int)o.cm_group;
-#pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int e = j * NT + tk;
-                    const V2<R> l = lam[swz(e)], q = phi[swz(e ^ (1 << lb))];
-                    double v;
-                    if (o.g == GEN_X) {
-                        v = (double)l.x * q.y - (double)l.y * q.x;
-                    } else {
-                        const double re = (double)l.x * q.x + (double)l.y * q.y;
-                        v = ((e >> lb) & 1) ? re : -re;
-                    }
-                    a += v;
-                }
             } else {
                 const int lb = (int)o.cm_group;
+                auto sum = [&](auto plain) {  // plain: no controls, so no index tests
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int e = j * NT + tk;
-                    const uint64_t gi = gk | pd.top[j];
-                    const V2<R> l = lam[swz(e)], q = phi[swz(e ^ (1 << lb))];
-                    double v;
-                    if (o.g == GEN_X) {
-                        v = (double)l.x * q.y - (double)l.y * q.x;
-                    } else {  // Y: (Y psi)[e] = +i q where bit lb of e is set, -i q where clear
-                        const double re = (double)l.x * q.x + (double)l.y * q.y;
-                        v = ((e >> lb) & 1) ? re : -re;
+                    for (int j = 0; j < 8; j++) {
+                        const int e = j * NT + tk;
+                        const V2<R> l = lam[swz(e)], q = phi[swz(e ^ (1 << lb))];
+                        double v;
+                        if (o.g == GEN_X) {
+                            v = (double)l.x * q.y - (double)l.y * q.x;
+                        } else {
+                            const double re = (double)l.x * q.x + (double)l.y * q.y;
+                            v = ((e >> lb) & 1) ? re : -re;
+                        }
+                        if constexpr (decltype(plain)::value)
+                            a += v;
+                        else
+                            a += (((gk | pd.top[j]) & o.cm_ext) == o.cm_ext) ? v : 0.0;
                     }
-                    a += ((gi & o.cm_ext) == o.cm_ext) ? v : 0.0;
-                }
+                };
+                if (o.cm_ext == 0)
+                    sum(std::true_type{});
+                else
+                    sum(std::false_type{});
             }
 #pragma unroll
             for (int kk = 0; kk < 8; kk++) acc[kk] = kk == k ? a : acc[kk];
         }
         const double t = wave_total8(acc, lane);
-        const int m = (((lane >> 5) & 1) << 2) | (((lane >> 4) & 1) << 1) | ((lane >> 3) & 1);
-        if ((lane & 7) == 0 && m < cn) red[m * 8 + wave] = t;
+        if ((lane & 7) == 0 && total8_of < cn) red[total8_of * 8 + wave] = t;
         __syncthreads();
         if (tid < cn) {
             double sum = 0.0;
-            for (int wv = 0; wv < (NT >> 6); wv++) sum += red[tid * 8 + wv];
+            for (int wv = 0; wv < waves; wv++) sum += red[tid * 8 + wv];
             partials[(uint64_t)ops[c0 + tid].flags * tiles + blockIdx.x] = sum;
         }
         __syncthreads();
     }
+}
+
+// pxmask of a stage's markers: bits 0 to 31 the columns of X and Y that any asks for, 32 to 47 the number of
+// markers on their own (they come first), 48 whether a Z is among the others; from 49 on, for each of
+// the others, 6 bits of its column, 3 bits of wavefront numbers that flip its sign, 1 bit: the sign is
+// that of its qubit's bit, outside the tile
+template <typename R>
+static void grad_info(FOpDev<R>* ops, FOpDev<R>* end, const int* local_of, int b) {
+    uint64_t info = 0;
+    for (FOpDev<R>* o = ops; o != end; o++) {
+        if (o->cm_ext != 0 || (sizeof(R) == 4 && o->g != GEN_Z)) {
+            info += 1ull << 32;
+            continue;
+        }
+        uint64_t at;
+        if (o->g == GEN_Z) {
+            info |= 1ull << 48;
+            const int lb = local_of[o->cm_group];
+            if (lb < 0)
+                at = 32 | (1u << 9);
+            else if (lb >= b - 3)
+                at = 33 + lb - (b - 3);
+            else if (lb < 6)
+                at = 36 + lb;
+            else
+                at = 32 | (1u << (lb - 6) << 6);
+        } else {
+            const int lb = (int)o->cm_group, g = std::min(lb / 3, 3);
+            at = 8 * g + (o->g == GEN_X ? 0 : 3) + lb - (g < 3 ? 3 * g : b - 3);
+            info |= 1ull << at;
+        }
+        o->pxmask = at << 49;
+    }
+    for (FOpDev<R>* o = ops; o != end; o++) o->pxmask |= info;
 }
 
 // Streaming accesses: the state is far larger than L2 and the MALL, and a pass touches each line
@@ -1035,9 +1157,10 @@ __device__ __forceinline__ void hscatter(const V2<R> (&v)[8], V2<R>* tile, int s
 
 // NS = 2: the reverse sweep, both states' tiles side by side in LDS (as k_fused_pass), gradient
 // stages evaluated from LDS between compute groups.
-// (two-state tiles fit two workgroups per CU at most, so that instantiation may use 256 registers)
+// (two-state tiles fit two workgroups per CU at most, so that instantiation may use 256 registers at
+// complex128, whose tiles have 256 threads, and 128 at complex64, where they have 512)
 template <typename R, int NS>
-__global__ void __launch_bounds__(NS == 1 ? 1024 : 512) k_fused_half(V2<R>* __restrict__ psi, V2<R>* __restrict__ psi1,
+__global__ void __launch_bounds__(NS == 1 ? 1024 : 512, NS == 2 && sizeof(R) == 4 ? 4 : 1) k_fused_half(V2<R>* __restrict__ psi, V2<R>* __restrict__ psi1,
                                                      const PassDesc pd, const FOpDev<R>* __restrict__ ops,
                                                      const unsigned char* __restrict__ runs,
                                                      double* __restrict__ partials, uint64_t tiles) {
@@ -1049,7 +1172,7 @@ __global__ void __launch_bounds__(NS == 1 ? 1024 : 512) k_fused_half(V2<R>* __re
     // after the tiles: the gradient stages' wavefront sums (NS = 2), then the global offsets of the
     // tile's high local bits (local index >> L)
     double* red = reinterpret_cast<double*>(tile + NS * T);
-    uint64_t* hi_tab = reinterpret_cast<uint64_t*>(red + (NS == 2 ? 64 : 0));
+    uint64_t* hi_tab = reinterpret_cast<uint64_t*>(red + (NS == 2 ? GRAD_RED : 0));
     const int L = pd.L;
     {
         // element e of the tile goes to LDS slot swz(e) (the swizzle is an involution). complex128:
@@ -1763,7 +1886,12 @@ static PassDesc encode_pass(const State& s, const FPass& p, std::vector<FOpDev<R
             pd.stage_mask |= 1u << gi;
             pd.gop[gi] = (int)h.size() - first;
             for (int j = 0; j < FUSE_GROUP_BITS; j++) pd.gbits[gi][j] = 0;
-            for (const FOpHost& o : G.ops) {
+            // markers that the split-row kernel evaluates on their own come first (see grad_stage8)
+            std::vector<FOpHost> markers(G.ops);
+            const auto own = [](const FOpHost& o) { return o.cm_ext != 0 || (sizeof(R) == 4 && o.g != GEN_Z); };
+            std::stable_partition(markers.begin(), markers.end(), own);
+            const size_t stage_first = h.size();
+            for (const FOpHost& o : markers) {
                 FOpDev<R> d{};
                 d.kind = F_GRAD;
                 d.g = o.g;
@@ -1778,6 +1906,7 @@ static PassDesc encode_pass(const State& s, const FPass& p, std::vector<FOpDev<R
                 slots.push_back(o.slot);
                 h.push_back(d);
             }
+            grad_info(h.data() + stage_first, h.data() + h.size(), local_of, b);
             continue;
         }
         for (int j = 0; j < gbn; j++) {
@@ -2048,7 +2177,8 @@ static void execute_typed(State& s, const std::vector<PlanItem>& plan, void* lam
         if constexpr (sizeof(R) == 8 || NS == 2) {
             const int hb_max = NS == 1 ? 13 : 12;  // at most 1024 / 512 threads
             if (s.split_rows && pd.b >= 10 && pd.b <= hb_max) {
-                const size_t lds_h = lds + ((size_t)1 << (pd.b - pd.L)) * sizeof(uint64_t);
+                const size_t lds_h = NS * ((size_t)1 << pd.b) * sizeof(V2<R>) + (NS == 2 ? GRAD_RED * sizeof(double) : 0) +
+                                     ((size_t)1 << (pd.b - pd.L)) * sizeof(uint64_t);
                 if (lds_h > 160 * 1024) throw Error(QFVM_ERR_RUNTIME, "split-row tile exceeds 160 KiB of LDS");
                 if (lds_h > 65536) allow_large_lds(reinterpret_cast<const void*>(&k_fused_half<R, NS>), s.device);
                 {
