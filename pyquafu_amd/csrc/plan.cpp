@@ -386,15 +386,16 @@ std::vector<Gate> collapse_dense_blocks(const std::vector<Gate>& gates, int k, i
 std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const FuseConfig& cfg) {
     const int b = std::min(cfg.tile_bits, n);
     const int gb = cfg.group_bits;
-    // a tile keeps at least one free slot when it does not hold every qubit, so the first waiting
-    // gate always fits and every pass makes progress
+    // a tile keeps at least one free slot when it does not hold every qubit, and gates that need more run
+    // by themselves, so the first waiting gate always fits and every pass makes progress
     const int L = b < n ? std::min(cfg.low_bits, b - 1) : b;
     const uint64_t all = n >= 64 ? ~0ull : ((1ull << n) - 1);
     // Layout-aware plans (cfg.layout, row-of-8 passes): qubit q sits at position phys[q] (inv is the
     // inverse); gates are planned on positions. At the end of every pass the tile qubits with the
     // nearest next non-diagonal use move into the L low positions, which every later tile holds, so
     // the next pass needs fewer new positions; passes without gates restore the identity at the end.
-    const bool lay = cfg.layout && b < n && gb == 3;
+    // A tile with one free slot cannot exchange two high positions, so it keeps every qubit in place.
+    const bool lay = cfg.layout && b - L >= 2 && b < n && gb == 3;
     std::vector<int> phys, inv;
     if (lay) {
         phys.resize((size_t)n);
@@ -406,8 +407,10 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
     std::vector<GInfo> info(gates.size());
     for (size_t i = 0; i < gates.size(); i++) {
         info[i] = info_of(gates[i]);
-        // row-of-8 groups hold a dense 2-target gate as one 4x4 op (both targets in one group)
-        if (gb == 3 && info[i].multi && gates[i].targets.size() == 2) {
+        // row-of-8 groups hold a dense 2-target gate as one 4x4 op (both targets in one group) where the
+        // tile has a slot for each target above the low qubits (with one free slot nothing moves)
+        if (gb == 3 && info[i].multi && gates[i].targets.size() == 2 &&
+            (b == n || b - L >= 2 || popc(info[i].N >> L) <= b - L)) {
             info[i].multi = false;
             info[i].dense2 = true;
         }
@@ -524,6 +527,7 @@ std::vector<PlanItem> plan_gates(const std::vector<Gate>& gates, int n, const Fu
             Q = newQ;
             done[i] = 1;
         }
+        if (groups.empty()) throw Error(QFVM_ERR_RUNTIME, "a fused pass cannot hold the next gate");
         // finalize: pad the tile to b qubits and every group to gb tile qubits. Matrix-core passes whose
         // qubits are out of place take misplaced positions with their qubits' homes first
         if (moved && cfg.mat)
