@@ -335,8 +335,8 @@ int qfvm_profile_json(qfvm_handle h, char* buf, int64_t cap, int64_t* len, int32
  *   "stagger_shift" the blockIdx bit that selects the delayed half (0..16)
  *   "mfma"        1 = (default) dense gates on 4 to 8 targets and, with "rows8" on, the groups of
  *                 complex128 one-state passes (2^9 to 2^13-amplitude tiles with 128-byte runs or
- *                 longer; gate lists that are mostly controlled phases keep the vector kernels where
- *                 those take less time) run on the matrix cores (FP64 MFMA at complex128, FP32 MFMA at
+ *                 longer; gate lists of a few gates, mostly X with controls or mostly controlled
+ *                 phases keep the vector kernels where those take less time) run on the matrix cores (FP64 MFMA at complex128, FP32 MFMA at
  *                 complex64), 0 = on the vector ALUs
  *   "dense_blocks" k (0 = off, or 4..8; default 5): qfvm_apply and qfvm_run (not qfvm_adjoint) on
  *                 states of 14 or more qubits with "mfma" on collapse runs of gates confined to at
@@ -369,7 +369,8 @@ int qfvm_set_option(qfvm_handle h, const char* key, int64_t value);
 
 /*
  * The execution plan qfvm_apply would run for `prog` on an n-qubit state, as JSON (host only, no
- * device needed; no counterpart in the reference). Fused passes list their tile qubits (positions),
+ * device needed; no counterpart in the reference). Fused passes say whether they run on the matrix
+ * cores ("mat") and list their tile qubits (positions),
  * "out_bit" (layout-aware plans: where each tile bit is stored; empty = in place) and, per group,
  * the ops in execution order: {"kind", "g", "g2", "cmg", "cme", "run", "m": [re, im] x 4, or x 16
  * for a 4x4 on group bits g and g2 (kind 9)}; other items

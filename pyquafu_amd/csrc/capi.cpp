@@ -1299,7 +1299,8 @@ int qfvm_plan_json(int32_t n, int32_t dtype, int32_t tile_bits, int32_t low_bits
             const PlanItem& it = plan[i];
             j += i ? ", " : "";
             if (it.fused) {
-                j += "{\"fused\": true, \"group_bits\": " + std::to_string(it.pass.group_bits) + ", \"Q\": [";
+                j += "{\"fused\": true, \"mat\": " + std::string(it.pass.mat ? "true" : "false") + ", \"group_bits\": " +
+                     std::to_string(it.pass.group_bits) + ", \"Q\": [";
                 for (size_t k = 0; k < it.pass.Q.size(); k++) j += (k ? ", " : "") + std::to_string(it.pass.Q[k]);
                 j += "], \"out_bit\": [";
                 for (size_t k = 0; k < it.pass.out_bit.size(); k++) j += (k ? ", " : "") + std::to_string(it.pass.out_bit[k]);

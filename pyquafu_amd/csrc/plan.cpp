@@ -927,6 +927,57 @@ FuseConfig circuit_config(const State& s, const std::vector<Gate>& gates) {
     return b >= 9 && b <= 13 && low >= 3 ? cfg : vec;
 }
 
+// Time of a plan in units of a complex128 vector pass that streams the state and computes little (8 us
+// at 16 qubits, 1.45 ms at 28): per pass its traffic and what its gates add. Fitted to 1247 gate lists of
+// 9 to 30 qubits (random dense gates, CX, H and CCX lists, CX chains, brickworks, rotations and CZ
+// rings, dense two-qubit gates, 8 to 12 n gates), each timed on both kinds of passes: the cheaper plan by
+// this is within 1% of the faster one on average, and at most 1.09 times the vector plan's time where
+// matrix-core passes for every list of 8 or more gates took up to 1.5 times it (CX lists, lists of a
+// few gates). States of 2^24 amplitudes stream from HBM; the passes of smaller ones wait for
+// their chain of gates instead, and those of up to 2^18 for little but their launch.
+static double plan_time(const std::vector<PlanItem>& plan, int n) {
+    struct Cost {
+        double vec, gate2, diag, x, run, member, gate4;  // a vector pass: its base and its ops
+        double mat, group, build;                        // a matrix-core pass, and the call's matrices
+        double single;                                   // a gate by itself
+    };
+    static constexpr Cost kSmall = {0.5, 0.053, 0.038, 0.023, 0.14, 0.012, 0.41, 0.755, 0.065, 0.13, 1.0};
+    static constexpr Cost kMid = {0.6, 0.07, 0.055, 0.035, 0.14, 0.006, 0.32, 0.98, 0.10, 0.23, 1.3};
+    static constexpr Cost kLarge = {1.0, 0.06, 0.04, 0.03, 0.03, 0.002, 0.12, 0.95, 0.21, 0.15, 0.9};
+    const Cost& c = n <= 18 ? kSmall : n <= 23 ? kMid : kLarge;
+    double t = 0.0;
+    bool any_mat = false;
+    for (const PlanItem& it : plan) {
+        if (!it.fused) {
+            t += c.single;
+            continue;
+        }
+        if (it.pass.mat) {
+            any_mat = true;
+            t += c.mat + c.group * (double)it.pass.groups.size();
+            continue;
+        }
+        double p = c.vec;
+        for (const FGroup& G : it.pass.groups) {
+            int last_run = 0;
+            for (const FOpHost& o : G.ops) {
+                if (o.run > 0) {
+                    p += c.member + (o.run > last_run ? c.run : 0.0);
+                    last_run = o.run;
+                } else if (o.kind == F_DENSE || o.kind == F_REAL) {
+                    p += c.gate2;
+                } else if (o.kind == F_DIAG || o.kind == F_PHASE) {
+                    p += c.diag;
+                } else {
+                    p += o.kind == F_DENSE4 ? c.gate4 : c.x;
+                }
+            }
+        }
+        t += std::max(1.0, it.pass.group_bits == 4 ? 1.3 * p : p);  // rows of 16: tiles of 2^9 amplitudes
+    }
+    return any_mat ? t + c.build : t;
+}
+
 std::vector<PlanItem> plan_circuit(const std::vector<Gate>& gates, int n, const FuseConfig& cfg) {
     if (!cfg.mat) return plan_gates(gates, n, cfg);
     FuseConfig v = cfg;
@@ -938,16 +989,27 @@ std::vector<PlanItem> plan_circuit(const std::vector<Gate>& gates, int n, const 
     // a handful of gates (the runs between noise channels) is over before its matrices are built (10 us)
     if (gates.size() < 8) return plan_gates(gates, n, v);
     std::vector<PlanItem> plan = plan_gates(gates, n, cfg);
-    // Gate lists that are mostly diagonal gates between qubits far apart (a QFT: every pair) need many
-    // groups, since a group depends on few outside qubits, while the vector kernels merge any number
-    // of them into one angle per row. Measured at 28 qubits, complex128: a matrix-core pass takes
-    // 1.6 ms plus 0.11 ms per group, a vector pass of a QFT 2.0 ms.
-    // Gates with many controls run one by one between matrix-core passes but inside vector passes.
-    size_t diag = 0, single = 0;
-    for (const Gate& g : gates) diag += info_of(g).N == 0;
+    // Lists of many gates of which a third or more are neither diagonal nor X (the vector kernels merge
+    // controlled phases into angles and X into relabelings) are faster on the matrix cores at every size
+    // timed, so the other plan is not made for them.
+    size_t diag = 0, heavy = 0, single = 0;
+    for (const Gate& g : gates) {
+        const bool d = info_of(g).N == 0;
+        diag += d;
+        heavy += !d && g.kind != G_SWAP;
+    }
     for (const PlanItem& it : plan) single += !it.fused && it.gate.kind != G_MULTI;
-    if (diag <= 2 * (gates.size() - diag) && single == 0) return plan;
+    if (gates.size() > 4 * (size_t)n && 3 * heavy >= gates.size() && single == 0) return plan;
     std::vector<PlanItem> vec = plan_gates(gates, n, v);
+    if (plan_time(plan, n) > plan_time(vec, n)) return vec;
+    if (diag <= 2 * (gates.size() - diag) && single == 0) return plan;
+    // Lists that are mostly diagonal gates between qubits far apart (a QFT: every pair) need many groups,
+    // since a group depends on few outside qubits, while the vector kernels merge any number of them into
+    // one angle per row, and phases in proportion (a QFT's) into one term of it, which a plan does not
+    // show. Gates with many controls run one by one between matrix-core passes but inside
+    // vector passes. So these lists need clearly fewer passes as well: a QFT takes 2.0 ms per vector pass
+    // at 28 qubits and 1.6 ms plus 0.11 per group on the matrix cores (10 against 23 ms in all; 22 qubits 257
+    // against 326 us).
     double cm = 0.0, cv = 0.0;
     for (const PlanItem& it : plan) cm += it.fused ? 1.0 + 0.07 * (double)it.pass.groups.size() : 1.0;
     for (const PlanItem& it : vec) cv += it.fused ? 1.25 : 1.0;
