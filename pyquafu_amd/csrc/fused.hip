@@ -36,7 +36,8 @@ struct PassDesc {
     int q[FUSE_MAX_TILE_BITS];  // global qubit of local bit k (ascending; q[k] = k for k < L)
     int ngroups;
     uint32_t stage_mask;        // bit gi: group gi is a gradient stage (two-state passes)
-    int gbits[FUSE_MAX_GROUPS][FUSE_GROUP_BITS];  // local bits of each group, ascending
+    int gbits[FUSE_MAX_GROUPS][FUSE_GROUP_BITS];  // local bits of each group, ascending; of a stage, [0]: its
+                                                   //   number of markers on their own (see grad_stage8)
     int gop[FUSE_MAX_GROUPS + 1];                  // op ranges in the op array
     uint64_t gpxm[FUSE_MAX_GROUPS][FUSE_GROUP_BITS];  // relabel masks at each group's end
     uint32_t gpxc[FUSE_MAX_GROUPS];                   // relabel constants at each group's end
@@ -451,7 +452,8 @@ __device__ __forceinline__ double wave_total8(const double (&a)[8], int lane) {
 //     and that sum signed by each of the top three bits and by each of its six lane bits; other tile
 //     bits are the wavefront's number, qubits outside the tile sign the whole.
 // Which sums a stage needs and where each marker finds its own comes with the op records (grad_info): a loop
-// over the records here is a chain of scalar loads that costs more than the sums.
+// over the records here is a chain of scalar loads that costs more than the sums. The `alone` markers on
+// their own come first.
 // Bound by the LDS reads. 24 qubits, 8 layers of 48 markers, reverse sweep at complex128 13.4 -> 12.3 ms
 // with it before grad_info and the wider runs of chosen qubits (default_low_bits), 9.5 ms with both; at
 // complex64 7.03 -> 6.65 ms.
@@ -460,13 +462,12 @@ __device__ __forceinline__ double wave_total8(const double (&a)[8], int lane) {
 constexpr int GRAD_RED = 42 * 8;
 template <typename R>
 __device__ void grad_stage8(const V2<R>* phi, const V2<R>* lam, uint64_t g_tid, const PassDesc& pd,
-                            const FOpDev<R>* __restrict__ ops, int cnt, double* red, double* __restrict__ partials,
-                            uint64_t tiles) {
+                            const FOpDev<R>* __restrict__ ops, int cnt, int alone, double* red,
+                            double* __restrict__ partials, uint64_t tiles) {
     const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6, waves = NT >> 6, b = pd.b;
     const int total8_of = (((lane >> 5) & 1) << 2) | (((lane >> 4) & 1) << 1) | ((lane >> 3) & 1);
     const uint64_t info = ops[0].pxmask;  // of the stage (grad_info)
     const uint32_t need = (uint32_t)info;
-    const int alone = (int)((info >> 32) & 0xffffu);  // markers on their own, which come first
     const bool z = (info >> 48) & 1u;
     for (int g = 0; g < 4; g++) {
         if (sizeof(R) == 4) break;
@@ -612,16 +613,17 @@ __device__ void grad_stage8(const V2<R>* phi, const V2<R>* lam, uint64_t g_tid, 
     }
 }
 
-// pxmask of a stage's markers: bits 0 to 31 the columns of X and Y that any asks for, 32 to 47 the number of
-// markers on their own (they come first), 48 whether a Z is among the others; from 49 on, for each of
-// the others, 6 bits of its column, 3 bits of wavefront numbers that flip its sign, 1 bit: the sign is
-// that of its qubit's bit, outside the tile
+// pxmask of a stage's markers: bits 0 to 31 the columns of X and Y that any asks for, 48 whether a Z is
+// among those with a column; from 49 on, for each of these, 6 bits of its column, 3 bits of wavefront
+// numbers that flip its sign, 1 bit: the sign is that of its qubit's bit, outside the tile. Returns the
+// number of markers on their own, which come first: a stage may hold any number of them.
 template <typename R>
-static void grad_info(FOpDev<R>* ops, FOpDev<R>* end, const int* local_of, int b) {
+static int grad_info(FOpDev<R>* ops, FOpDev<R>* end, const int* local_of, int b) {
     uint64_t info = 0;
+    int alone = 0;
     for (FOpDev<R>* o = ops; o != end; o++) {
         if (o->cm_ext != 0 || (sizeof(R) == 4 && o->g != GEN_Z)) {
-            info += 1ull << 32;
+            alone++;
             continue;
         }
         uint64_t at;
@@ -644,6 +646,7 @@ static void grad_info(FOpDev<R>* ops, FOpDev<R>* end, const int* local_of, int b
         o->pxmask = at << 49;
     }
     for (FOpDev<R>* o = ops; o != end; o++) o->pxmask |= info;
+    return alone;
 }
 
 // Streaming accesses: the state is far larger than L2 and the MALL, and a pass touches each line
@@ -1215,7 +1218,7 @@ __global__ void __launch_bounds__(NS == 1 ? 1024 : 512, NS == 2 && sizeof(R) == 
         if constexpr (NS == 2) {
             if ((pd.stage_mask >> gi) & 1u) {
                 grad_stage8<R>(tile, tile + T, base | local_to_global(tid, pd), pd, ops + pd.gop[gi],
-                               pd.gop[gi + 1] - pd.gop[gi], red, partials, tiles);
+                               pd.gop[gi + 1] - pd.gop[gi], pd.gbits[gi][0], red, partials, tiles);
                 continue;  // grad_stage8 ends with a barrier
             }
         }
@@ -1906,7 +1909,7 @@ static PassDesc encode_pass(const State& s, const FPass& p, std::vector<FOpDev<R
                 slots.push_back(o.slot);
                 h.push_back(d);
             }
-            grad_info(h.data() + stage_first, h.data() + h.size(), local_of, b);
+            pd.gbits[gi][0] = grad_info(h.data() + stage_first, h.data() + h.size(), local_of, b);
             continue;
         }
         for (int j = 0; j < gbn; j++) {
