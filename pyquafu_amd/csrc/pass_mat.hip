@@ -292,6 +292,38 @@ __device__ __forceinline__ void mat_product(const unsigned char* lds, const MatC
     }
 }
 
+// The same product entry by entry, skipping the matrix's zeros (see k_pass_mat); `at` is filled as well.
+__device__ __forceinline__ void mat_product_sparse(const unsigned char* lds, const MatCursor& c, const MatGroup& G, int lane,
+                                                   int (&at)[4], d4 (&acc)[4]) {
+    const int kq = lane >> 4, kx0 = G.kx[0], kx1 = G.kx[1];
+#pragma unroll
+    for (int cb = 0; cb < 4; cb++) {
+        at[cb] = c.sl ^ ((cb & 1) ? c.cb0 : 0) ^ ((cb & 2) ? c.cb1 : 0);
+        const int row = at[cb] ^ ((kq & 1) ? kx0 : 0) ^ ((kq & 2) ? kx1 : 0);  // slot of member 0
+        const double* a = c.mat - lane * 4 + ((cb & 2) ? c.vcb : 0);
+        d4 y = {0, 0, 0, 0};
+#pragma unroll 1
+        for (int m = 0; m < 8; m++) {
+            const double2 x = *reinterpret_cast<const double2*>(
+                lds + (row ^ ((m & 1) ? c.mx : 0) ^ ((m & 2) ? kx0 : 0) ^ ((m & 4) ? kx1 : 0)));
+#pragma unroll
+            for (int r = 0; r < 2; r++) {  // member 2 kq + r of the result
+                const double* w = a + (8 * r + kq + 16 * (m >> 1)) * 4 + ((m & 1) << 1);
+                const double re = w[0], im = -w[1];
+                if (re != 0.0) {
+                    y[2 * r] = fma(re, x.x, y[2 * r]);
+                    y[2 * r + 1] = fma(re, x.y, y[2 * r + 1]);
+                }
+                if (im != 0.0) {
+                    y[2 * r] = fma(-im, x.y, y[2 * r]);
+                    y[2 * r + 1] = fma(im, x.x, y[2 * r + 1]);
+                }
+            }
+        }
+        acc[cb] = y;
+    }
+}
+
 __device__ __forceinline__ void mat_put(double2* p, double2 v, int nt) {
     typedef double d2 __attribute__((ext_vector_type(2)));
     const d2 w = {v.x, v.y};
@@ -321,9 +353,23 @@ __device__ __forceinline__ void store_tile(double2* __restrict__ psi, const unsi
     __builtin_amdgcn_s_setprio(0);
 }
 
+// every row belongs to one wavefront, whose reads precede its writes
+__device__ __forceinline__ void mat_scatter(unsigned char* lds, const int (&at)[4], int mx, const d4 (&acc)[4]) {
+#pragma unroll
+    for (int cb = 0; cb < 4; cb++) {
+        *reinterpret_cast<double2*>(lds + at[cb]) = make_double2(acc[cb][0], acc[cb][1]);
+        *reinterpret_cast<double2*>(lds + (at[cb] ^ mx)) = make_double2(acc[cb][2], acc[cb][3]);
+    }
+}
+
 // One tile per workgroup of 2^(b-3) threads; wavefront w holds rows 64 w .. 64 w + 63 of every group
 // (in the group's own row order) as four column blocks. `nt`: the state is far larger than the
 // caches, so its lines are loaded and stored with the non-temporal hint.
+// The matrix cores multiply every entry, so an infinity or a NaN reaches all members of its row (0 * inf),
+// though gates as X, CX, CZ and diagonal ones only move or scale amplitudes. Such a row has no finite
+// product from then on; so the last group's products tell, and before anything is stored the tile is loaded
+// again and multiplied without the matrices' zeros (a flag after the tile; checking each group's
+// products took 5% of the 30-qubit circuit).
 __global__ void __launch_bounds__(1024) k_pass_mat(double2* __restrict__ psi, const MatPass pd,
                                                    const double* __restrict__ mats, int nt) {
     extern __shared__ unsigned char lds[];
@@ -331,12 +377,14 @@ __global__ void __launch_bounds__(1024) k_pass_mat(double2* __restrict__ psi, co
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint64_t base = mat_base(blockIdx.x, pd);
     const uint64_t g_sw = base | mat_local(mat_slot(tid), pd);
+    int* again = reinterpret_cast<int*>(lds + (size_t)NT * 128);
     __builtin_amdgcn_s_setprio(2);
     if (nt)
         load_tile<2>(psi, lds, pd, g_sw, NT, wave);
     else
         load_tile<0>(psi, lds, pd, g_sw, NT, wave);
     __builtin_amdgcn_s_setprio(0);
+    if (tid == 0) *again = 0;
     MatCursor cur{};
     if (pd.ngroups > 0) cur = mat_open(pd.g[0], base, wave, lane, mats);
     __builtin_amdgcn_s_waitcnt(0);
@@ -347,13 +395,28 @@ __global__ void __launch_bounds__(1024) k_pass_mat(double2* __restrict__ psi, co
         mat_product(lds, cur, at, acc);
         const int mx = cur.mx;
         cur = mat_open(pd.g[gi + 1 < pd.ngroups ? gi + 1 : gi], base, wave, lane, mats);  // arrives over the barrier
-        // every row belongs to one wavefront, whose reads precede its writes
-#pragma unroll
-        for (int cb = 0; cb < 4; cb++) {
-            *reinterpret_cast<double2*>(lds + at[cb]) = make_double2(acc[cb][0], acc[cb][1]);
-            *reinterpret_cast<double2*>(lds + (at[cb] ^ mx)) = make_double2(acc[cb][2], acc[cb][3]);
+        mat_scatter(lds, at, mx, acc);
+        if (gi + 1 == pd.ngroups) {
+            const bool finite = __builtin_isfinite(acc[0][0]) & __builtin_isfinite(acc[1][0]) &
+                                __builtin_isfinite(acc[2][0]) & __builtin_isfinite(acc[3][0]);
+            if (!__all(finite) && lane == 0) *again = 1;
         }
         lds_barrier();
+    }
+    if (__builtin_amdgcn_readfirstlane(*again)) {
+        __syncthreads();
+        load_tile<0>(psi, lds, pd, g_sw, NT, wave);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+#pragma unroll 1
+        for (int gi = 0; gi < pd.ngroups; gi++) {
+            int at[4];
+            d4 acc[4];
+            const MatCursor c = mat_open(pd.g[gi], base, wave, lane, mats);
+            mat_product_sparse(lds, c, pd.g[gi], lane, at, acc);
+            mat_scatter(lds, at, c.mx, acc);
+            __syncthreads();
+        }
     }
     store_tile(psi, lds, pd, base | mat_local(tid, pd), tid, NT, nt);
 }
@@ -563,7 +626,7 @@ void execute_mat_plan(State& s, const std::vector<PlanItem>& plan) {
                 continue;
             }
             const MatPass& pd = passes[k++];
-            const size_t lds = ((size_t)1 << pd.b) * sizeof(double2);
+            const size_t lds = ((size_t)1 << pd.b) * sizeof(double2) + sizeof(double2);  // and k_pass_mat's flag
             const unsigned threads = (1u << pd.b) >> 3;
             if (lds > 65536) allow_large_lds(reinterpret_cast<const void*>(&k_pass_mat), s.device);
             const int nt = s.size * sizeof(double2) > (256ull << 20) ? 1 : 0;
