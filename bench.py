@@ -10,8 +10,8 @@ Printed (one JSON line):
   roofline       the dominant kernel's algorithmic bytes per launch / its mean HIP-event duration,
                  against MI355X's 8 TB/s HBM peak; stream_ref times a plain in-place streaming kernel
                  (torch neg_) over a buffer of the state's size, and frac_of_stream = achieved / its rate
-  layout         the same circuit with the layout-aware planner (option "layout"): time per step,
-                 fused passes, speedup over the default planner
+  layout         the same circuit with the layout-aware planner (option "layout") off and on: time per
+                 step, fused passes, speedup over the default (on for matrix-core passes)
   merge_1q       runs of U3 layers with one-qubit runs merged (default) and not (option merge_1q)
   gate_equiv     the unfused per-gate byte model (sum over gates of 2 * 16 B * 2^(n - controls)) /
                  step time: comparable with the CPU, may exceed the HBM peak once gates are fused
@@ -644,25 +644,27 @@ def main(argv=None) -> int:
         "energy_h0.7": float(sum(tfim_vals[:n]) + 0.7 * sum(tfim_vals[n:])),
     }
 
-    # the layout-aware planner (option "layout") on the same circuit: fewer passes, more gates each
-    dev.set_option("layout", 1)
-    dev.apply(prog)
-    dev.synchronize()
-    dev.profile(reset=True)
-    t0 = time.perf_counter()
-    for _ in range(args.steps):
+    # the layout-aware planner (option "layout") on the same circuit, off and on: fewer passes, more
+    # gates each (by default it is on for matrix-core passes and off for the others)
+    layout_leg = {"option": "layout"}
+    for on in (0, 1):
+        dev.set_option("layout", on)
         dev.apply(prog)
-    dev.synchronize()
-    dt_lay = (time.perf_counter() - t0) / args.steps
-    lay_prof = dev.profile(reset=True)
-    dev.set_option("layout", 0)
-    layout_leg = {
-        "option": "layout",
-        "ms_per_step": round(dt_lay * 1e3, 3),
-        "fused_passes_per_step": lay_prof.get("fused_pass", {}).get("launches", 0) / args.steps,
-        "speedup_vs_default": round(dt / dt_lay, 4),
-        "pass_model_GBps": round(sum(v["bytes"] for v in lay_prof.values()) / args.steps / dt_lay / 1e9, 2),
-    }
+        dev.synchronize()
+        dev.profile(reset=True)
+        t0 = time.perf_counter()
+        for _ in range(args.steps):
+            dev.apply(prog)
+        dev.synchronize()
+        dt_lay = (time.perf_counter() - t0) / args.steps
+        lay_prof = dev.profile(reset=True)
+        layout_leg["on" if on else "off"] = {
+            "ms_per_step": round(dt_lay * 1e3, 3),
+            "fused_passes_per_step": lay_prof.get("fused_pass", {}).get("launches", 0) / args.steps,
+            "speedup_vs_default": round(dt / dt_lay, 4),
+            "pass_model_GBps": round(sum(v["bytes"] for v in lay_prof.values()) / args.steps / dt_lay / 1e9, 2),
+        }
+    dev.set_option("layout", -1)
 
     # option merge_1q (runs of one-qubit gates merged, default on) on runs of U3 layers
     runs_leg = {"workload": f"{n}q {args.dtype} workloads.u3_runs: 8 layers of U3 on every qubit, CX(2i, 2i+1) "

@@ -326,8 +326,8 @@ int qfvm_profile_json(qfvm_handle h, char* buf, int64_t cap, int64_t* len, int32
  *                 in other places (the tile's addresses stay the same), so that the qubits the next
  *                 passes act on sit in the low positions every tile holds; fewer passes per circuit,
  *                 and the qubits are back in order at the end of each call, so the state between
- *                 calls is always in the standard order. 1 = on, 0 = off; by default it is on for
- *                 matrix-core passes (see "mfma") and off for the others
+ *                 calls is always in the standard order. 1 = on, 0 = off; -1 (default) = on for
+ *                 matrix-core passes (see "mfma"), off for the others
  *   "stream"      1 = persistent fused-pass kernel that prefetches the next tile (complex128,
  *                 one-state passes of 2^11..2^13-amplitude tiles, when split_rows does not apply),
  *                 0 = one workgroup per tile
@@ -377,7 +377,7 @@ int qfvm_set_option(qfvm_handle h, const char* key, int64_t value);
  * carry the gate on the positions it runs at. Lets the planner's reordering be checked without a
  * GPU. Arguments of 0 pick the defaults, as for qfvm_set_option, except dense_blocks: 0 plans
  * without collapsing runs, 4..8 collapses them as option "dense_blocks" does (at any n), with
- * dense_min_gates (0 = 24); layout = 1 plans as option "layout" does. One-qubit runs are merged
+ * dense_min_gates (0 = 24); layout plans as option "layout" does (-1: its default). One-qubit runs are merged
  * as with option "merge_1q" on (its default). Items outside passes carry
  * their matrix ("m": the 2x2, or the 2^k x 2^k of a dense gate, row-major).
  */

@@ -107,16 +107,16 @@ SIGNATURES = {
 
 
 def plan_json(prog: Program, n: int, dtype: str = "c128", tile_bits: int = 0, low_bits: int = 0,
-              max_groups: int = 0, pass_cost: int = 0, layout: bool = False, dense_blocks: int = 0,
+              max_groups: int = 0, pass_cost: int = 0, layout: int = 0, dense_blocks: int = 0,
               dense_min_gates: int = 0) -> dict:
     """The fused execution plan the engine would run for `prog` (host only; no GPU needed);
-    `layout`, `dense_blocks` and `dense_min_gates` plan as the options of those names do (with
-    `dense_blocks` = 0, the default here, no run is collapsed)."""
+    `layout`, `dense_blocks` and `dense_min_gates` plan as the options of those names do (their defaults
+    here: every qubit stays in place, -1 plans as the engine does by default, and no run is collapsed)."""
     import json  # pylint: disable=import-outside-toplevel
 
     cp, keep = as_cprogram(prog)
     ln = ctypes.c_int64(0)
-    args = (int(n), _DTYPES[dtype], int(tile_bits), int(low_bits), int(max_groups), int(pass_cost), int(bool(layout)),
+    args = (int(n), _DTYPES[dtype], int(tile_bits), int(low_bits), int(max_groups), int(pass_cost), int(layout),
             int(dense_blocks), int(dense_min_gates), ctypes.byref(cp))
     check(lib().qfvm_plan_json(*args, None, 0, ctypes.byref(ln)))
     buf = ctypes.create_string_buffer(ln.value + 1)

@@ -1227,7 +1227,7 @@ int qfvm_set_option(qfvm_handle h, const char* key, int64_t value) {
         } else if (k == "rows8_c64") {
             s->rows8_c64 = value != 0;
         } else if (k == "layout") {
-            s->layout = value != 0;
+            s->layout = value == -1 ? -1 : value != 0;
         } else if (k == "plan_cache") {
             s->plan_cache_on = value != 0;
             if (!value) s->plan_cache.reset();
@@ -1283,7 +1283,7 @@ int qfvm_plan_json(int32_t n, int32_t dtype, int32_t tile_bits, int32_t low_bits
         if (dense_blocks) gates = collapse_dense_blocks(gates, dense_blocks, dense_min_gates > 0 ? dense_min_gates : 24);
         tmp.tile_bits = tile_bits;
         tmp.low_bits = low_bits;
-        tmp.layout = layout != 0;
+        tmp.layout = layout == -1 ? -1 : layout != 0;
         FuseConfig cfg = circuit_config(tmp, gates);  // with default options, as qfvm_apply
         if (tile_bits > 0 && tile_bits < cfg.tile_bits) cfg.tile_bits = tile_bits;
         cfg.max_groups = max_groups > 0 ? max_groups : 12;

@@ -45,3 +45,30 @@ def test_a_layer_that_saves_a_pass_takes_the_matrix_cores(n):
     for q in range(12):
         b.add(GENERAL, [q], matrix=random_unitary(2, rng)) if q % 2 else b.add(H, [q])
     assert _mat(b.program(n_qubits=n), n)
+
+
+@pytest.mark.parametrize("n", [14, 20])
+def test_layout_option_defaults(n):
+    """-1, the default of option "layout": on where the list runs on the matrix cores, off elsewhere."""
+    brick = compile_circuit(workloads.random_u3_cx(n, 6, 4, seed=5, measure=False))
+    plans = [_native.plan_json(brick, n, layout=v) for v in (-1, 1, 0)]
+    assert plans[0] == plans[1] != plans[2]
+    qft = compile_circuit(workloads.qft(20, 12345))
+    plans = [_native.plan_json(qft, 20, layout=v) for v in (-1, 0, 1)]
+    assert plans[0] == plans[1] != plans[2]
+
+
+@pytest.mark.gpu
+def test_layout_option_set_back():
+    n = 20
+    prog = compile_circuit(workloads.random_u3_cx(n, 6, 4, seed=5, measure=False))
+    dev = _native.DeviceState(n, "c128")
+    passes = []
+    for value in (None, 0, 1, -1):
+        if value is not None:
+            dev.set_option("layout", value)
+        dev.profile(reset=True)
+        dev.apply(prog)
+        passes.append(dev.profile(reset=True)["fused_pass"]["launches"])
+    dev.close()
+    assert passes[0] == passes[2] == passes[3] != passes[1]
