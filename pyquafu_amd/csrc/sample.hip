@@ -318,15 +318,22 @@ __global__ void __launch_bounds__(256) k_seq_descend(const V2<R>* __restrict__ p
 // thread, in order, each from the end of the one before and the composed pairs between. Blocks that cannot
 // change S (all p zero, or below half an ulp of both binades of the interval) are the identity and not
 // special. Exactness does not rest on the margin: every pair's use is checked against the exact S (its
-// binade, no carry out of it), and a check that fails, more than SEQ_SPECIALS special blocks, or sums that
-// are not finite send the call to the chunk loop.
+// binade, no carry out of it). A block that cannot change S needs no such check: its 32 terms are each
+// below 2^-53 of the lower of its two binades, so it can hold only one of their ends, and S is in
+// one of the two unless it is off by a factor of nearly two, where N 2^-53 bounds it. A check that fails,
+// more than SEQ_SPECIALS special blocks, or sums that are not finite hand over to the chunk loop, which
+// goes on from the first block concerned: the ends before it are exact. (A tail of equal terms drifts
+// from A beyond the margin, all roundings being the same. One amplitude of probability 1 - 10^-k and such a
+// tail, k = 5 to 11: 24 qubits at most 0.43 ms, 26 at most 1.02, 27 at most 1.86, where starting over
+// took up to 1.03, 1.57 and 2.31 ms and the chunk loop alone takes 0.87, 1.13 and 1.53. A special block costs 0.4
+// us, so more than 256 of them are better left to the loop: k = 9 at 24 qubits 0.70 -> 0.43 ms.)
 // What bounds it: two reads of the state, and some 40 us of launches up to 18 qubits; the chunk loop
 // reads once, so it stays the better one for larger states, whose reads outweigh its waits (SEQ_BYTES:
 // 28 qubits at complex128 1.84 -> 1.63 ms; two reads of 29 qubits would take 3.2, one and the waits 2.7).
 // Measured for one shot of a random complex128 state: 12 qubits 268 -> 48 us, 18 qubits 469 -> 52 us, 24
 // qubits 818 -> 151 us, 26 qubits 1.11 -> 0.45 ms.
 constexpr uint64_t SEQ_BYTES = 4ull << 30;
-constexpr unsigned SEQ_SPECIALS = 1024;
+constexpr unsigned SEQ_SPECIALS = 256;
 constexpr int SEQ_IDENTITY = -32768;  // exponent entry of a block that keeps S
 constexpr double SEQ_TINY = 0x1p-1000;  // below it every block that changes S is special
 
@@ -339,8 +346,8 @@ struct SeqSpecial {
     Xfer before;  // pairs between the special block before and this one
 };
 struct SeqFast {
-    unsigned total;  // special blocks
-    int failed;
+    uint64_t bad;    // first block whose end is not known to be exact (NONE: all are)
+    uint64_t total;  // special blocks
 };
 
 __device__ __forceinline__ SegX seg_compose(SegX f, SegX g) {
@@ -365,7 +372,7 @@ __global__ void __launch_bounds__(256) k_seq_mass(const V2<R>* __restrict__ psi,
     constexpr int TE = TILE_BLOCKS * SB;
     __shared__ double wsum[4];
     const int tid = threadIdx.x;
-    if (blockIdx.x == 0 && tid == 0) *st = SeqFast{0, 0};
+    if (blockIdx.x == 0 && tid == 0) *st = SeqFast{NONE, 0};
     const uint64_t at = (uint64_t)blockIdx.x * TE;
     double a = 0.0;
 #pragma unroll
@@ -405,6 +412,15 @@ __global__ void __launch_bounds__(SCAN_GROUP) k_seq_mass_prefix(const double* __
     __syncthreads();
     for (int j = 0; j < SCAN_GROUP / 64; j++) ex += wbefore[j] + (j < wv ? wtot[j] : 0.0);
     if (first + tid < ntiles) pre[first + tid] = ex;
+}
+
+// reports the first of a wavefront's blocks (ascending over its lanes) that is not good
+__device__ __forceinline__ void seq_report(bool good, uint64_t block, SeqFast* st) {
+    const uint64_t m = __ballot(!good);
+    // (blocks past a reported one skip the atomic: one address would serialise them all)
+    if (m && (int)(threadIdx.x & 63) == __ffsll((unsigned long long)m) - 1 &&
+        block < *reinterpret_cast<volatile uint64_t*>(&st->bad))
+        atomicMin(reinterpret_cast<unsigned long long*>(&st->bad), (unsigned long long)block);
 }
 
 // Pairs of every block for its binade (bx, its exponent in be), the tile's special blocks (mask) and its
@@ -464,9 +480,9 @@ __global__ void __launch_bounds__(256) k_seq_pairs(const V2<R>* __restrict__ psi
     const double lo = a0 * (1.0 - eps), hi = a1 * (1.0 + eps);
     bool special = false;
     int e = SEQ_IDENTITY;
-    if (!(a1 <= 1.7976931348623157e308)) {
-        st->failed = 1;
-    } else if (q > 0.0) {
+    const bool finite = a1 <= 1.7976931348623157e308;
+    seq_report(finite, tb0 + tid / (SB / RUN), st);
+    if (finite && q > 0.0) {
         if (lo < SEQ_TINY) {
             special = true;
         } else {
@@ -621,11 +637,7 @@ __global__ void __launch_bounds__(256) k_seq_resolve(const V2<R>* __restrict__ p
     constexpr int BATCH = 128;
     __shared__ double p[BATCH * SB];
     __shared__ Xfer before[BATCH];
-    const unsigned total = st->total;
-    if (total > SEQ_SPECIALS) {
-        if (threadIdx.x == 0) st->failed = 1;
-        return;
-    }
+    const unsigned total = (unsigned)min(st->total, (uint64_t)SEQ_SPECIALS);
     double s = 0.0;
     for (unsigned k0 = 0; k0 < total; k0 += BATCH) {
         const unsigned n = min((unsigned)BATCH, total - k0);
@@ -652,17 +664,18 @@ __global__ void __launch_bounds__(256) k_seq_ends(const Xfer* __restrict__ bx, c
                                                   double* __restrict__ B, SeqFast* st) {
     const int lane = threadIdx.x & 63;
     const uint64_t t = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= ntiles || st->total > SEQ_SPECIALS) return;
+    if (t >= ntiles) return;  // whole wavefronts
     const uint64_t m = mask[t];
     const SegX pre = tpre[t];
     const Xfer x = seg_block(bx, pre, m, t, lane, nblk);
     const uint64_t cb = t * TILE_BLOCKS + lane;
-    if (cb >= nblk) return;
+    const bool in = cb < nblk;
     const unsigned k = pre.count + (unsigned)__popcll(m & ((2ull << lane) - 1));  // special blocks up to this one
-    const double s = k > 0 ? ends[k - 1] : 0.0;
-    const int want = be[cb];
+    const bool known = k <= SEQ_SPECIALS;
+    const double s = k > 0 && known ? ends[k - 1] : 0.0;
+    const int want = in ? be[cb] : SEQ_IDENTITY;
     double end = s;
-    bool good = s <= 1.7976931348623157e308;
+    bool good = known && s <= 1.7976931348623157e308;
     if (s > 0.0 && good) {
         int e;
         int64_t mm;
@@ -671,14 +684,35 @@ __global__ void __launch_bounds__(256) k_seq_ends(const Xfer* __restrict__ bx, c
     } else if (want != SEQ_IDENTITY) {
         good = false;
     }
-    if (!good) st->failed = 1;
-    B[cb] = end;
+    seq_report(good || !in, cb, st);
+    if (in) B[cb] = end;
 }
 
+// scratch of the chunk loop (sample_typed); the block ends come first, as in sample_fast
+struct SeqScratch {
+    size_t b, bx, tx, gx, st, u, o;
+    uint64_t chunk_max;
+    SeqScratch(uint64_t nblk, int64_t shots) {
+        auto align = [](size_t x) { return (x + 255) & ~size_t(255); };
+        chunk_max = std::min<uint64_t>(nblk, 1ull << 24);
+        const uint64_t tiles_max = (chunk_max + TILE_BLOCKS - 1) / TILE_BLOCKS;
+        const uint64_t groups_max = (tiles_max + SCAN_GROUP - 1) / SCAN_GROUP;
+        b = align(nblk * sizeof(double));
+        bx = align(chunk_max * sizeof(Xfer));
+        tx = align(tiles_max * sizeof(Xfer));
+        gx = align(groups_max * sizeof(Xfer));
+        st = align(sizeof(SeqStatus));
+        u = align((size_t)shots * sizeof(double));
+        o = align((size_t)shots * sizeof(uint64_t));
+    }
+    size_t bytes() const { return b + bx + 2 * tx + gx + st + u + o; }
+};
 
-// Block ends and shots of a state of up to SEQ_BYTES. False: nothing was written, the chunk loop has to run.
+// Block ends and shots of a state of up to SEQ_BYTES. Returns the first block whose end could not be
+// told (NONE: all were, and host_out is written); the ends before it are at the start of the scratch
+// and *last is the last of them.
 template <typename R>
-static bool sample_fast(State& s, const double* host_u, int64_t shots, uint64_t* host_out) {
+static uint64_t sample_fast(State& s, const double* host_u, int64_t shots, uint64_t* host_out, double* last) {
     const uint64_t nblk = s.size / SB;
     const uint64_t ntiles = (nblk + TILE_BLOCKS - 1) / TILE_BLOCKS;
     const uint64_t ngroups = (ntiles + SCAN_GROUP - 1) / SCAN_GROUP;
@@ -697,12 +731,13 @@ static bool sample_fast(State& s, const double* host_u, int64_t shots, uint64_t*
     // copies the uniforms there while the scan runs. 26 qubits: 100000 shots 533 -> 494 us, 200000 shots 651 -> 583.
     const bool few = shots <= (1 << 20);
     const size_t ou = part(few ? 0 : (size_t)shots * sizeof(double)), oo = part(few ? 0 : (size_t)shots * sizeof(uint64_t));
-    char* base = reinterpret_cast<char*>(s.ensure_scratch(bytes));
+    // (the chunk loop may go on with it, and a larger scratch would lose the ends)
+    char* base = reinterpret_cast<char*>(s.ensure_scratch(std::max(bytes, SeqScratch(nblk, shots).bytes())));
     const size_t per = few ? (size_t)shots : 0;
     double* pin = s.ensure_pinned(sizeof(SeqFast) + per * (sizeof(double) + sizeof(uint64_t)));
     SeqFast* hst = reinterpret_cast<SeqFast*>(pin);
-    static_assert(sizeof(SeqFast) == sizeof(double), "pinned layout");
-    double* hu = pin + 1;
+    static_assert(sizeof(SeqFast) == 2 * sizeof(double), "pinned layout");
+    double* hu = pin + 2;
     uint64_t* ho = reinterpret_cast<uint64_t*>(hu + per);
     auto at = [&](size_t o) { return base + o; };
     double* B = reinterpret_cast<double*>(at(oB));
@@ -750,44 +785,45 @@ static bool sample_fast(State& s, const double* host_u, int64_t shots, uint64_t*
     }
     QFVM_HIP(hipMemcpyAsync(hst, st, sizeof(SeqFast), hipMemcpyDeviceToHost, s.stream));
     QFVM_HIP(hipStreamSynchronize(s.stream));
-    if (hst->failed) return false;
+    if (hst->bad != NONE) {
+        const uint64_t bad = hst->bad;
+        *last = 0.0;
+        if (bad > 0) {
+            QFVM_HIP(hipMemcpyAsync(pin, B + bad - 1, sizeof(double), hipMemcpyDeviceToHost, s.stream));
+            QFVM_HIP(hipStreamSynchronize(s.stream));
+            *last = *pin;
+        }
+        return bad;
+    }
     if (few)
         std::copy(ho, ho + shots, host_out);
     else {
         QFVM_HIP(hipMemcpyAsync(host_out, dout, (size_t)shots * sizeof(uint64_t), hipMemcpyDeviceToHost, s.stream));
         QFVM_HIP(hipStreamSynchronize(s.stream));
     }
-    return true;
+    return NONE;
 }
 
+// from > 0: the ends of the blocks before it are at hand (sample_fast), S = `at` at the last of them
 template <typename R>
-static void sample_typed(State& s, const double* host_u, int64_t shots, uint64_t* host_out) {
+static void sample_typed(State& s, const double* host_u, int64_t shots, uint64_t* host_out, uint64_t from = 0,
+                         double at = 0.0) {
     const int n = s.n;
     const uint64_t size = s.size;
     const int w = size >= (uint64_t)SB ? SB : (int)size;
     const uint64_t nblk = size / (uint64_t)w;
-    const uint64_t chunk_max = std::min<uint64_t>(nblk, 1ull << 24);
-    const uint64_t tiles_max = (chunk_max + TILE_BLOCKS - 1) / TILE_BLOCKS;
-    const uint64_t groups_max = (tiles_max + SCAN_GROUP - 1) / SCAN_GROUP;
-    auto align = [](size_t b) { return (b + 255) & ~size_t(255); };
-    const size_t b_bytes = align(nblk * sizeof(double));
-    const size_t bx_bytes = align(chunk_max * sizeof(Xfer));
-    const size_t tx_bytes = align(tiles_max * sizeof(Xfer));
-    const size_t gx_bytes = align(groups_max * sizeof(Xfer));
-    const size_t st_bytes = align(sizeof(SeqStatus));
-    const size_t u_bytes = align((size_t)shots * sizeof(double));
-    const size_t o_bytes = align((size_t)shots * sizeof(uint64_t));
-    char* base = reinterpret_cast<char*>(
-        s.ensure_scratch(b_bytes + bx_bytes + 2 * tx_bytes + gx_bytes + st_bytes + u_bytes + o_bytes));
+    const SeqScratch sz(nblk, shots);
+    const uint64_t chunk_max = sz.chunk_max;
+    char* base = reinterpret_cast<char*>(s.ensure_scratch(sz.bytes()));
     double* B = reinterpret_cast<double*>(base);
-    Xfer* bx = reinterpret_cast<Xfer*>(base + b_bytes);
-    Xfer* tx = reinterpret_cast<Xfer*>(base + b_bytes + bx_bytes);
-    Xfer* tpre = reinterpret_cast<Xfer*>(base + b_bytes + bx_bytes + tx_bytes);
-    Xfer* gx = reinterpret_cast<Xfer*>(base + b_bytes + bx_bytes + 2 * tx_bytes);
-    char* tail = base + b_bytes + bx_bytes + 2 * tx_bytes + gx_bytes;
+    Xfer* bx = reinterpret_cast<Xfer*>(base + sz.b);
+    Xfer* tx = reinterpret_cast<Xfer*>(base + sz.b + sz.bx);
+    Xfer* tpre = reinterpret_cast<Xfer*>(base + sz.b + sz.bx + sz.tx);
+    Xfer* gx = reinterpret_cast<Xfer*>(base + sz.b + sz.bx + 2 * sz.tx);
+    char* tail = base + sz.b + sz.bx + 2 * sz.tx + sz.gx;
     SeqStatus* st = reinterpret_cast<SeqStatus*>(tail);
-    double* du = reinterpret_cast<double*>(tail + st_bytes);
-    uint64_t* dout = reinterpret_cast<uint64_t*>(tail + st_bytes + u_bytes);
+    double* du = reinterpret_cast<double*>(tail + sz.st);
+    uint64_t* dout = reinterpret_cast<uint64_t*>(tail + sz.st + sz.u);
     SeqStatus* hst = reinterpret_cast<SeqStatus*>(s.ensure_pinned(sizeof(SeqStatus)));
     const V2<R>* psi = reinterpret_cast<const V2<R>*>(s.psi);
     auto read_status = [&] {
@@ -799,14 +835,20 @@ static void sample_typed(State& s, const double* host_u, int64_t shots, uint64_t
         KernelScope ks(s, "sample_scan", (double)size * s.amp_bytes() + (double)nblk * sizeof(double));
         hipLaunchKernelGGL(k_seq_init, dim3(1), dim3(64), 0, s.stream, st);
         QFVM_LAUNCHED();
-        hipLaunchKernelGGL(k_first_nonzero<R>, dim3(grid_for(size, 256, 2048)), dim3(256), 0, s.stream, psi, size,
-                           st);
-        QFVM_LAUNCHED();
-        read_status();
-        const uint64_t b0 = hst->first == NONE ? nblk : hst->first / (uint64_t)w;
-        if (b0 > 0) launch_zero(s, B, b0 * sizeof(double));
+        uint64_t b0 = 0;
         uint64_t next = nblk;
         double S = 0.0;
+        if (from > 0) {
+            next = from;
+            S = at;
+        } else {
+            hipLaunchKernelGGL(k_first_nonzero<R>, dim3(grid_for(size, 256, 2048)), dim3(256), 0, s.stream, psi, size,
+                               st);
+            QFVM_LAUNCHED();
+            read_status();
+            b0 = hst->first == NONE ? nblk : hst->first / (uint64_t)w;
+            if (b0 > 0) launch_zero(s, B, b0 * sizeof(double));
+        }
         double rate = 0.0;  // growth of S per block over the last evaluated span
         auto finish = [&](uint64_t start, uint64_t end, double s_start, int seq_only) {
             hipLaunchKernelGGL(k_seq_finish<R>, dim3(1), dim3(64), 0, s.stream, psi, start, end, s_start, seq_only, w, B,
@@ -818,7 +860,7 @@ static void sample_typed(State& s, const double* host_u, int64_t shots, uint64_t
             rate = next > start ? (S - s_start) / (double)(next - start) : 0.0;
         };
         int singles = 0;  // consecutive blocks replayed alone because a crossing was expected there
-        if (b0 < nblk) finish(b0, b0 + 1, 0.0, 1);
+        if (from == 0 && b0 < nblk) finish(b0, b0 + 1, 0.0, 1);
         const uint64_t min_chunk = 1ull << 12;
         while (next < nblk) {
             if (!std::isfinite(S)) {  // inf / NaN amplitudes: the sum stays where it is
@@ -881,14 +923,18 @@ static void sample_typed(State& s, const double* host_u, int64_t shots, uint64_t
 
 void sample_sequential_rule(State& s, const double* host_u, int64_t shots, uint64_t* host_out) {
     if (shots <= 0) return;
-    if (s.size >= (uint64_t)SB && (uint64_t)s.size * s.amp_bytes() <= SEQ_BYTES &&
-        (s.dtype == QFVM_C128 ? sample_fast<double>(s, host_u, shots, host_out)
-                              : sample_fast<float>(s, host_u, shots, host_out)))
-        return;
+    uint64_t from = 0;
+    double at = 0.0;
+    if (s.size >= (uint64_t)SB && (uint64_t)s.size * s.amp_bytes() <= SEQ_BYTES) {
+        from = s.dtype == QFVM_C128 ? sample_fast<double>(s, host_u, shots, host_out, &at)
+                                    : sample_fast<float>(s, host_u, shots, host_out, &at);
+        if (from == NONE) return;
+        if (!(at >= SEQ_TINY)) from = 0;  // the loop finds the first nonzero block itself
+    }
     if (s.dtype == QFVM_C128)
-        sample_typed<double>(s, host_u, shots, host_out);
+        sample_typed<double>(s, host_u, shots, host_out, from, at);
     else
-        sample_typed<float>(s, host_u, shots, host_out);
+        sample_typed<float>(s, host_u, shots, host_out, from, at);
 }
 
 }  // namespace qfvm
