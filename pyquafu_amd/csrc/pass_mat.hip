@@ -277,7 +277,7 @@ __device__ __forceinline__ void mat_gather(const unsigned char* lds, const MatCu
 // The first and the last two k steps are summed apart and added: the partial sums are half as long, and
 // with them the product's rounding (error of the state after 40 layers on 16 qubits 2.12e-15 with
 // one sum, 1.95e-15 with two, 1.90e-15 with four; 1.89e-15 on the vector kernels). Two blocks at a time two
-// sums cost nothing (30 qubits, 10 layers 258.2 and 258.5 ms; four sums 268).
+// sums cost nothing (30 qubits, 10 layers: 260.0 ms with one, 254.9 with two; four take 4% more).
 __device__ __forceinline__ bool mat_pair(unsigned char* lds, const MatRows& w, int mx, int cb, const d4& a) {
     d4 sum[2][2];
 #pragma unroll
@@ -300,16 +300,15 @@ __device__ __forceinline__ bool mat_pair(unsigned char* lds, const MatRows& w, i
     return fin;
 }
 
-// The same product entry by entry, skipping the matrix's zeros (see k_pass_mat); `at` is filled as well.
-__device__ __forceinline__ void mat_product_sparse(const unsigned char* lds, const MatCursor& c, const MatGroup& G, int lane,
-                                                   int (&at)[4], d4 (&acc)[4]) {
+// The same products entry by entry, skipping the matrix's zeros (see k_pass_mat), stored.
+__device__ __forceinline__ void mat_sparse(unsigned char* lds, const MatCursor& c, const MatGroup& G, int lane) {
     const int kq = lane >> 4, kx0 = G.kx[0], kx1 = G.kx[1];
-#pragma unroll
+#pragma unroll 1
     for (int cb = 0; cb < 4; cb++) {
-        at[cb] = c.sl ^ ((cb & 1) ? c.cb0 : 0) ^ ((cb & 2) ? c.cb1 : 0);
-        const int row = at[cb] ^ ((kq & 1) ? kx0 : 0) ^ ((kq & 2) ? kx1 : 0);  // slot of member 0
+        const int at = c.sl ^ ((cb & 1) ? c.cb0 : 0) ^ ((cb & 2) ? c.cb1 : 0);
+        const int row = at ^ ((kq & 1) ? kx0 : 0) ^ ((kq & 2) ? kx1 : 0);  // slot of member 0
         const double* a = c.mat - lane * 4 + ((cb & 2) ? c.vcb : 0);
-        d4 y = {0, 0, 0, 0};
+        double2 y[2] = {{0.0, 0.0}, {0.0, 0.0}};
 #pragma unroll 1
         for (int m = 0; m < 8; m++) {
             const double2 x = *reinterpret_cast<const double2*>(
@@ -319,16 +318,18 @@ __device__ __forceinline__ void mat_product_sparse(const unsigned char* lds, con
                 const double* w = a + (8 * r + kq + 16 * (m >> 1)) * 4 + ((m & 1) << 1);
                 const double re = w[0], im = -w[1];
                 if (re != 0.0) {
-                    y[2 * r] = fma(re, x.x, y[2 * r]);
-                    y[2 * r + 1] = fma(re, x.y, y[2 * r + 1]);
+                    y[r].x = fma(re, x.x, y[r].x);
+                    y[r].y = fma(re, x.y, y[r].y);
                 }
                 if (im != 0.0) {
-                    y[2 * r] = fma(-im, x.y, y[2 * r]);
-                    y[2 * r + 1] = fma(im, x.x, y[2 * r + 1]);
+                    y[r].x = fma(-im, x.y, y[r].x);
+                    y[r].y = fma(im, x.x, y[r].y);
                 }
             }
         }
-        acc[cb] = y;
+        // (the wavefront has read the block's rows; no other block holds them)
+        *reinterpret_cast<double2*>(lds + at) = y[0];
+        *reinterpret_cast<double2*>(lds + (at ^ c.mx)) = y[1];
     }
 }
 
@@ -392,34 +393,36 @@ __global__ void __launch_bounds__(1024) k_pass_mat(double2* __restrict__ psi, co
         MatRows w;
         mat_gather(lds, cur, w);
         const int mx = cur.mx;
-        d4 a2 = cur.a;
-        if (cur.vcb) a2 = *reinterpret_cast<const d4*>(cur.mat + cur.vcb);
-        bool finite = mat_pair(lds, w, mx, 0, cur.a);
-        cur = mat_open(pd.g[gi + 1 < pd.ngroups ? gi + 1 : gi], base, wave, lane, mats);  // arrives over the barrier
-        finite = mat_pair(lds, w, mx, 2, a2) & finite;
+        bool finite;
+        const MatGroup& next = pd.g[gi + 1 < pd.ngroups ? gi + 1 : gi];  // its matrix arrives over the barrier
+        if (cur.vcb == 0) {  // one matrix for the wavefront
+            const d4 a = cur.a;
+            finite = mat_pair(lds, w, mx, 0, a);
+            cur = mat_open(next, base, wave, lane, mats);
+            finite = mat_pair(lds, w, mx, 2, a) & finite;
+        } else {
+            const d4 a = *reinterpret_cast<const d4*>(cur.mat + cur.vcb);
+            finite = mat_pair(lds, w, mx, 0, cur.a);
+            cur = mat_open(next, base, wave, lane, mats);
+            finite = mat_pair(lds, w, mx, 2, a) & finite;
+        }
         if (gi + 1 == pd.ngroups && !__all(finite) && lane == 0) *again = 1;
         lds_barrier();
     }
+    int t = tid;
+    asm volatile("" : "+v"(t));  // (offsets are formed anew: kept over the groups, they would not fit the registers)
     if (__builtin_amdgcn_readfirstlane(*again)) {
         __syncthreads();
-        load_tile<0>(psi, lds, pd, g_sw, NT, wave);
+        load_tile<0>(psi, lds, pd, base | mat_local(mat_slot(t), pd), NT, wave);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
 #pragma unroll 1
         for (int gi = 0; gi < pd.ngroups; gi++) {
-            int at[4];
-            d4 acc[4];
-            const MatCursor c = mat_open(pd.g[gi], base, wave, lane, mats);
-            mat_product_sparse(lds, c, pd.g[gi], lane, at, acc);
-#pragma unroll
-            for (int cb = 0; cb < 4; cb++) {
-                *reinterpret_cast<double2*>(lds + at[cb]) = make_double2(acc[cb][0], acc[cb][1]);
-                *reinterpret_cast<double2*>(lds + (at[cb] ^ c.mx)) = make_double2(acc[cb][2], acc[cb][3]);
-            }
+            mat_sparse(lds, mat_open(pd.g[gi], base, wave, lane, mats), pd.g[gi], lane);
             __syncthreads();
         }
     }
-    store_tile(psi, lds, pd, base | mat_local(tid, pd), tid, NT, nt);
+    store_tile(psi, lds, pd, base | mat_local(t, pd), t, NT, nt);
 }
 
 // ------------------------------------------------------------------------------------------------
