@@ -646,23 +646,24 @@ def main(argv=None) -> int:
 
     # the layout-aware planner (option "layout") on the same circuit, off and on: fewer passes, more
     # gates each (by default it is on for matrix-core passes and off for the others)
-    layout_leg = {"option": "layout"}
+    lay_steps = min(args.steps, 3)
+    layout_leg = {"option": "layout", "steps": lay_steps}
     for on in (0, 1):
         dev.set_option("layout", on)
         dev.apply(prog)
         dev.synchronize()
         dev.profile(reset=True)
         t0 = time.perf_counter()
-        for _ in range(args.steps):
+        for _ in range(lay_steps):
             dev.apply(prog)
         dev.synchronize()
-        dt_lay = (time.perf_counter() - t0) / args.steps
+        dt_lay = (time.perf_counter() - t0) / lay_steps
         lay_prof = dev.profile(reset=True)
         layout_leg["on" if on else "off"] = {
             "ms_per_step": round(dt_lay * 1e3, 3),
-            "fused_passes_per_step": lay_prof.get("fused_pass", {}).get("launches", 0) / args.steps,
+            "fused_passes_per_step": lay_prof.get("fused_pass", {}).get("launches", 0) / lay_steps,
             "speedup_vs_default": round(dt / dt_lay, 4),
-            "pass_model_GBps": round(sum(v["bytes"] for v in lay_prof.values()) / args.steps / dt_lay / 1e9, 2),
+            "pass_model_GBps": round(sum(v["bytes"] for v in lay_prof.values()) / lay_steps / dt_lay / 1e9, 2),
         }
     dev.set_option("layout", -1)
 
