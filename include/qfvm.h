@@ -168,7 +168,7 @@ int qfvm_expect_paulis(qfvm_handle h, const char* chars, const int32_t* pos, con
  * qfvm_expect_paulis without any allocation. No counterpart in the reference: it is for callers that
  * cannot allocate device or pinned memory (code under HIP graph capture setup, tight serving loops,
  * harnesses that forbid hipMalloc). Same terms, same results (the same kernels, the same summation
- * order) as qfvm_expect_paulis, but every scratch byte lives in a fixed 530 KiB device array that
+ * order) as qfvm_expect_paulis, but every scratch byte lives in a fixed 1426 KiB device array that
  * the library holds per GPU until the process ends: at most 256 terms per call (more ->
  * QFVM_ERR_VALUE). Calls on one GPU share that array, so calls that overlap on one GPU (two threads,
  * two handles) race; serialise them. The state must not be modified concurrently either.
@@ -306,8 +306,8 @@ int qfvm_profile_json(qfvm_handle h, char* buf, int64_t cap, int64_t* len, int32
  *   "tile_bits"   qubits per fused tile b (4..14; 0 = default: 12 for matrix-core passes, else 11 for
  *                 complex128, 12 for complex64;
  *                 the adjoint's two-state sweep uses b - 1 of an explicit value, 11 / 12 by default)
- *   "low_bits"    low qubits always in a tile L (0 = default: 4 for matrix-core passes, 3 at complex128
- *                 up to 25 qubits; else 5 for one-state passes, 6 for two-state)
+ *   "low_bits"    low qubits always in a tile L (0 = default: matrix-core passes 3 up to 25 qubits, else
+ *                 4; other one-state passes 5; two-state passes 3 at complex128, 6 at complex64)
  *   "max_groups"  register groups (of 3 or 4 qubits) per fused pass (1..24, default 12)
  *   "pass_cost"   compute budget of one fused pass in quarter dense-gate units (0 = default)
  *   "split_rows"  1 = (default) complex128 one-state passes of 2^10..2^13-amplitude tiles and the

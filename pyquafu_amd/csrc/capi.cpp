@@ -306,7 +306,6 @@ struct Runner {
             for (size_t j = 0; j < q.size(); j++) creg[(*c)[j]] = (int32_t)((m >> j) & 1);
     }
 
-    // a noise channel on one qubit (include/qfvm.h: QFVM_OP_KRAUS / QFVM_OP_UCHAN)
     // the qubit and the matrices of a well-formed channel; false if the op is not one
     bool channel_matrices(const qfvm_op& op, int* q, std::vector<std::array<cd, 4>>& m) const {
         if (op.n_qubits != 1 || !p->idx || op.q_off < 0 || op.q_off >= p->n_idx || op.body < 1 || op.body > 64) return false;
@@ -358,6 +357,7 @@ struct Runner {
         reduce_populations(s, run_qubits, run_pop);
     }
 
+    // a noise channel on one qubit (include/qfvm.h: QFVM_OP_KRAUS / QFVM_OP_UCHAN), ops[at]
     void channel(const qfvm_op& op, int64_t at, int64_t end) {
         std::vector<int> q = op_list(p, op.q_off, op.n_qubits);
         check_qubits(s, q);

@@ -116,7 +116,8 @@ inline int mat_ext(int b) { return b - 8 < MAT_MAX_EXT ? b - 8 : MAT_MAX_EXT; }
 // pass against 39% at 2^13, 33-qubit QFT 234 vs 249 ms). Contiguous runs of 32 amplitudes for one
 // state; for two, 64 at complex64 and 8 (whole lines) at complex128, which leaves 8 chosen qubits: 24
 // qubits, 8 layers of rotations and a CZ ring take 10 reverse passes instead of 15 (16.1 -> 12.1 ms with
-// fuller gradient stages; 26 qubits 61 -> 54).
+// fuller gradient stages). 4 layers, against runs of 64 and the stages and forward passes of that
+// time: 11 qubits 0.75 of the time, 16 0.74, 20 0.68, 24 0.66, 26 0.71, 28 0.69, 30 0.70 (434 ms).
 inline int default_tile_bits(int dtype, int /*states*/) { return dtype == QFVM_C128 ? 11 : 12; }
 inline int default_low_bits(int dtype, int states) { return states == 1 ? 5 : dtype == QFVM_C128 ? 3 : 6; }
 

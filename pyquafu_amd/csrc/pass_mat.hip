@@ -14,10 +14,11 @@
 // scatters them as whole amplitudes.
 //
 // What bounds it: the matrix cores take 2 cycles per amplitude and group on each of the 1024 SIMDs,
-// 0.87 ms per group and 2^30 amplitudes, beside 6.2 ms for the pass's memory traffic; the vector ALUs
-// only form LDS addresses. Measured on the 30-qubit, 10-layer benchmark circuit: 264 ms in 28 passes of 5
-// groups against 317 ms in 43 passes on the gate-by-gate kernel; 20 qubits, 20 layers 0.50 against
-// 1.10 ms. The gate-by-gate kernel (k_pass8) spends 0.22 ms per dense gate in vector
+// 0.87 ms per group and 2^30 amplitudes, beside 6.2 ms for the pass's memory traffic, and the two
+// overlap only in part. Counters of the 30-qubit, 10-layer benchmark circuit, means over 28 passes of 5 groups
+// and 9.1 ms (3.8 TB/s): matrix cores busy 49% of the cycles, vector instructions 20%, LDS 27% (a quarter of
+// that bank conflicts), HBM traffic 1.001 times the state's. Its passes take 255 ms, against 317 ms
+// in 43 passes on the gate-by-gate kernel; 20 qubits, 20 layers 0.50 against 1.10 ms. The gate-by-gate kernel (k_pass8) spends 0.22 ms per dense gate in vector
 // instructions that hide less. complex64 keeps the vector kernels, whose roundings its results are
 // compared by.
 #include <algorithm>

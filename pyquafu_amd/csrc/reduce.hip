@@ -355,6 +355,9 @@ __global__ void __launch_bounds__(RED_BLOCK) k_term_sums(const double* __restric
 // (complex64) chosen qubits: 3 reads for the fields of 27 to 30 qubits, where the tiles of general
 // strings (2^11 amplitudes, runs of 32, one accumulator per term) take 4 or 5. Measured on 27 qubits at
 // complex128, 27 ZZ bonds and 27 X fields: 2.62 ms -> 1.31 ms; 27 Z terms alone one read of 0.36 ms, 5.9 TB/s.
+// Counters at 30 qubits: the pass with the strings 4.0 ms (4.3 TB/s) with the LDS busy 49% of the cycles and the
+// vector ALUs 46%, passes with flips alone 3.5 to 4.7 ms (by where their qubits sit) with 17% each; every
+// pass reads the state once.
 constexpr int FT_BITS = 12;        // tile bits; smaller states are padded with zeros
 constexpr int FT_THREADS = 1 << (FT_BITS - 3);
 constexpr unsigned FT_GRID = 512;  // two workgroups per CU
@@ -799,12 +802,14 @@ void queue_expectations(State& s, const PauliHost* terms, int n_terms, double* o
 }
 
 // Allocation-free expectations (qfvm_expect_paulis_noalloc). Its scratch is this file-scope device
-// array: per-workgroup partials, the wide-term fallback's partials and the results, 530 KiB. Every
+// array: per-workgroup partials, the wide-term fallback's partials and the results, 1.4 MiB. Every
 // GPU the library runs on holds its own copy until the process ends, and every call on that GPU
 // shares it (calls that overlap on one GPU race). Host code never names the array in a kernel
 // argument or copy: it uses the address hipGetSymbolAddress returns, resolved once per device with
 // that device current.
 constexpr size_t NOALLOC_DOUBLES = EXPECT_PARTIALS + RED_PARTIALS + EXPECT_BATCH;
+// (include/qfvm.h tells the caller its size)
+static_assert(NOALLOC_DOUBLES * sizeof(double) / 1024 == 1426, "the documented size of the fixed scratch");
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 
 static double* noalloc_scratch(int device) {
