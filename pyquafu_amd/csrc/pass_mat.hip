@@ -369,8 +369,13 @@ __device__ __forceinline__ void store_tile(double2* __restrict__ psi, const unsi
 // The matrix cores multiply every entry, so an infinity or a NaN reaches all members of its row (0 * inf),
 // though gates as X, CX, CZ and diagonal ones only move or scale amplitudes. Such a row has no finite
 // product from then on; so the last group's products tell, and before anything is stored the tile is loaded
-// again and multiplied without the matrices' zeros (a flag after the tile; checking each group's
-// products took 5% of the 30-qubit circuit).
+// again and multiplied without the matrices' zeros (a flag after the tile; correcting each group's products
+// on the spot took 5% of the 30-qubit circuit).
+// LARGE (states of 2^24 amplitudes and more): wavefronts whose blocks take one matrix and those with two have
+// code of their own, and only the last group tests its products: 28 qubits, 6 layers 32.2 -> 31.2 ms, 26
+// qubits 7.08 -> 6.84. Smaller states wait for each tile's chain of groups instead, and the shorter code is
+// the faster one there (16 qubits, 3 layers 75.1 us against 77.2).
+template <bool LARGE>
 __global__ void __launch_bounds__(1024) k_pass_mat(double2* __restrict__ psi, const MatPass pd,
                                                    const double* __restrict__ mats, int nt) {
     extern __shared__ unsigned char lds[];
@@ -396,18 +401,19 @@ __global__ void __launch_bounds__(1024) k_pass_mat(double2* __restrict__ psi, co
         const int mx = cur.mx;
         bool finite;
         const MatGroup& next = pd.g[gi + 1 < pd.ngroups ? gi + 1 : gi];  // its matrix arrives over the barrier
-        if (cur.vcb == 0) {  // one matrix for the wavefront
+        if (LARGE && cur.vcb == 0) {  // one matrix for the wavefront
             const d4 a = cur.a;
             finite = mat_pair(lds, w, mx, 0, a);
             cur = mat_open(next, base, wave, lane, mats);
             finite = mat_pair(lds, w, mx, 2, a) & finite;
         } else {
-            const d4 a = *reinterpret_cast<const d4*>(cur.mat + cur.vcb);
+            d4 a = cur.a;
+            if (LARGE || cur.vcb) a = *reinterpret_cast<const d4*>(cur.mat + cur.vcb);
             finite = mat_pair(lds, w, mx, 0, cur.a);
             cur = mat_open(next, base, wave, lane, mats);
             finite = mat_pair(lds, w, mx, 2, a) & finite;
         }
-        if (gi + 1 == pd.ngroups && !__all(finite) && lane == 0) *again = 1;
+        if ((!LARGE || gi + 1 == pd.ngroups) && !__all(finite) && lane == 0) *again = 1;
         lds_barrier();
     }
     int t = tid;
@@ -633,10 +639,11 @@ void execute_mat_plan(State& s, const std::vector<PlanItem>& plan) {
             const MatPass& pd = passes[k++];
             const size_t lds = ((size_t)1 << pd.b) * sizeof(double2) + sizeof(double2);  // and k_pass_mat's flag
             const unsigned threads = (1u << pd.b) >> 3;
-            if (lds > 65536) allow_large_lds(reinterpret_cast<const void*>(&k_pass_mat), s.device);
+            const auto fn = s.n >= 24 ? k_pass_mat<true> : k_pass_mat<false>;
+            if (lds > 65536) allow_large_lds(reinterpret_cast<const void*>(fn), s.device);
             const int nt = s.size * sizeof(double2) > (256ull << 20) ? 1 : 0;
             KernelScope ks(s, "fused_pass", 2.0 * (double)s.size * sizeof(double2));
-            hipLaunchKernelGGL(k_pass_mat, dim3((unsigned)(1ull << (s.n - pd.b))), dim3(threads), lds, s.stream,
+            hipLaunchKernelGGL(fn, dim3((unsigned)(1ull << (s.n - pd.b))), dim3(threads), lds, s.stream,
                                reinterpret_cast<double2*>(s.psi), pd, mats, nt);
             QFVM_LAUNCHED();
         }

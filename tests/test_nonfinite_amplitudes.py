@@ -67,3 +67,38 @@ def test_nonfinite_amplitudes_stay_in_place(n, mixing, value):
     # the others do not depend on the marked ones: as in the run without them, to rounding (entries of a
     # group's matrix are products of at most 5 n unit phases; a result adds up at most 16 terms)
     assert np.abs(got - clean)[~marked].max() < 1e-13
+
+
+# states of 2^24 amplitudes and more take a kernel instance of their own
+def test_nonfinite_amplitudes_of_large_states():
+    n = 24
+    rng = np.random.Generator(np.random.PCG64(24))
+    b = ProgramBuilder()
+    at = rng.choice(1 << n, 5, replace=False)
+    marked = at.copy()
+    for k in range(5 * n):
+        q = [int(x) for x in rng.choice(n, 2, replace=False)]
+        if k % 3 == 0:
+            b.add(GENERAL, q[:1], matrix=np.array([[0, 1j], [1, 0]]))
+            marked ^= 1 << q[0]
+        elif k % 3 == 1:
+            b.add(CX, q, n_ctrl=1)
+            marked ^= ((marked >> q[0]) & 1) << q[1]
+        else:
+            b.add(CP, q, n_ctrl=1, param=0.3)
+    prog = b.program(n_qubits=n)
+    psi = np.full(1 << n, 2.0 ** (-n / 2), complex)
+    dev = _native.DeviceState(n, "c128")
+    dev.load(psi)
+    dev.apply(prog)
+    clean = dev.store()
+    psi[at] = [np.inf, -np.inf, np.nan, complex(0, np.inf), np.inf]
+    dev.load(psi)
+    dev.profile(reset=True)
+    dev.apply(prog)
+    got = dev.store()
+    assert "mat_build" in dev.profile()
+    dev.close()
+    bad = ~np.isfinite(got)
+    assert np.array_equal(np.flatnonzero(bad), np.sort(marked))
+    assert np.abs(got - clean)[~bad].max() < 1e-13
